@@ -66,6 +66,7 @@ struct Dual {
 
   // the face arithmetic's helpers (blk.h, k_flux.h) for dual arguments
   friend __device__ __forceinline__ Dual tdiv(const Dual &a, const Dual &b) { return a / b; }
+  friend __device__ __forceinline__ Dual xdiv(const Dual &a, const Dual &b) { return a / b; }
   friend __device__ __forceinline__ Dual tsqrt(const Dual &a) {
     Dual r;
     r.v = ::sqrt(a.v);

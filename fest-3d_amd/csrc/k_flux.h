@@ -29,13 +29,32 @@
 
 namespace fest {
 
-// FP64: the IEEE operations.  FP32 (the mixed-precision mode): the
+// The compiler's FP64 quotient: v_rcp_f64, two Newton steps, the quotient and
+// its remainder correction -- wrapped in v_div_scale, v_div_fmas and
+// v_div_fixup, which rescale operands near the ends of the exponent range.
+// The wrapper costs 3 of 11 instructions and runs every quotient of a thread
+// through VCC one after the other.  qdiv is the same sequence without it: the
+// same bits wherever b, 1/b and the quotient are normal numbers, as they are
+// for the face arithmetic's quotients (|b| from 1e-28, the WENO weights, to
+// 1e64).  Not for quotients that may be 0/0 or x/0: those take NaN here
+// (bmuscl_cell divides by plain differences and keeps a / b).
+__device__ __forceinline__ double qdiv(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// FP64: correctly rounded.  FP32 (the mixed-precision mode): the
 // hardware reciprocal and square root (v_rcp_f32, v_sqrt_f32, 1 ulp), whose
 // error is far below the FP32 face arithmetic's own.
 __device__ __forceinline__ double tsqrt(double x) { return sqrt(x); }
 __device__ __forceinline__ float tsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ double tdiv(double a, double b) { return a / b; }
+__device__ __forceinline__ double tdiv(double a, double b) { return qdiv(a, b); }
 __device__ __forceinline__ float tdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+// quotients whose divisor may be zero
+__device__ __forceinline__ double xdiv(double a, double b) { return a / b; }
+__device__ __forceinline__ float xdiv(float a, float b) { return tdiv(a, b); }
 __device__ __forceinline__ double tabs(double x) { return fabs(x); }
 __device__ __forceinline__ float tabs(float x) { return __builtin_fabsf(x); }
 
@@ -64,10 +83,10 @@ struct FaceMath {
     const T phi = T(1.0), kappa = T(1.) / T(3.);
     T fd = up - u0;
     T bd = u0 - um;
-    T r = tdiv(fd, bd);
+    T r = xdiv(fd, bd);
     T psi1 = fmx(T(0.), fmn(fmn(2 * r, (2 + r) / T(3.)), T(2.)));
     psi1 = (1 - (1 - psi1) * sw);
-    r = tdiv(bd, fd);
+    r = xdiv(bd, fd);
     T psi2 = fmx(T(0.), fmn(fmn(2 * r, (2 + r) / T(3.)), T(2.)));
     psi2 = (1 - (1 - psi2) * sw);
     upv = u0 + T(0.25) * phi * (((T(1.) - kappa) * psi1 * bd) + ((T(1.) + kappa) * psi2 * fd));
@@ -256,6 +275,60 @@ struct FaceMath {
       }
       if constexpr (recon == 1 || recon == 2) {
         if (ax.pb) R = w(3) - (ax.pdR * (w(3) - R));
+      }
+    }
+  }
+
+  // whether face n takes a boundary rule of face_states
+  template <int RECON>
+  static __device__ __forceinline__ bool edge_face(const Blk &b, int d, int n, int N) {
+    if (RECON == 0 || (n > 2 && n < N - 1)) return false;
+    const int minbc = b.bc[2 * d], maxbc = b.bc[2 * d + 1];
+    const bool bmin = minbc < 0 && minbc != -10, bmax = maxbc < 0 && maxbc != -10;
+    return (bmin && n <= (b.ppm_flag ? 2 : 1)) || (bmax && n >= (b.ppm_flag ? N - 1 : N));
+  }
+  // face_states of a face away from the boundary rules, without a branch:
+  // the stencil loads of one variable can be in flight while another's
+  // arithmetic runs, and the two cells' common differences are formed once
+  template <int RECON, typename Q>
+  static __device__ __forceinline__ void inner_states(const Blk &b, int d, int l, const Q *u, long s, const Aux &ax,
+                                                      T &L, T &R) {
+    auto w = [u, s](int m) { return T(u[(long)(m - 3) * s]); };
+    const int sw = (l >= 5) ? b.tlim[d] : b.lim[d];
+    T dummy;
+    if constexpr (RECON == 0) {
+      L = w(2);
+      R = w(3);
+    } else if constexpr (RECON == 1) {
+      const T w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4);
+      muscl_cell(w1, w2, w3, sw, L, dummy, b.valb);
+      muscl_cell(w2, w3, w4, sw, dummy, R, b.valb);
+      if (ax.pb) {
+        L = w2 + (ax.pdL * (L - w2));
+        R = w3 - (ax.pdR * (w3 - R));
+      }
+    } else if constexpr (RECON == 2) {
+      const T w0 = w(0), w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4), w5 = w(5);
+      const T f0 = ppm_face(w0, w1, w2, w3), f1 = ppm_face(w1, w2, w3, w4), f2 = ppm_face(w2, w3, w4, w5);
+      T lo = f0, up = f1;
+      if (b.lim[d] == 1) ppm_extrema(w2, up, lo);
+      L = up;
+      lo = f1;
+      up = f2;
+      if (b.lim[d] == 1) ppm_extrema(w3, up, lo);
+      R = lo;
+      if (ax.pb) {
+        L = w2 + (ax.pdL * (L - w2));
+        R = w3 - (ax.pdR * (w3 - R));
+      }
+    } else {
+      const T w0 = w(0), w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4), w5 = w(5);
+      if constexpr (RECON == 3) {
+        L = weno_up(w0, w1, w2, w3, w4);
+        R = weno_lo(w1, w2, w3, w4, w5);
+      } else {
+        L = weno_nm(w0, w1, w2, w3, w4, ax.A[0], ax.A[1], ax.A[2], ax.A[3], true);
+        R = weno_nm(w1, w2, w3, w4, w5, ax.A[1], ax.A[2], ax.A[3], ax.A[4], false);
       }
     }
   }
@@ -627,14 +700,22 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int store_c
       else M::pb_factors(b, n, N, qsrc + 4 * b.nc + c, s, ax);
     }
     if constexpr (RECON == 4) M::nm_blends(b.vol + c, s, ax);
+    // FP64 j and k sweeps: the boundary rules apart, the other faces without
+    // a branch.  At 256x128x128 (SST, WENO5) flux_j 482 -> 409 us, flux_k 479
+    // -> 408 us; the i sweep, whose stencils come from LDS, loses by it (439
+    // -> 466 us), and FP32 keeps the one form its results are defined by.
+    constexpr bool split = D != 0 && std::is_same<T, double>::value;
+    if (!split || M::template edge_face<RECON>(b, D, n, N)) {
 #pragma unroll
-    for (int l = 0; l < nv; ++l) {
-      if constexpr (D == 0) {
-        M::template face_states<RECON>(b, D, n, N, l, lds_row + l * (FLUX_I_SPAN + 5), 1, ax, qL[l], qR[l]);
-      } else {
-        const QS *u = qsrc + (long)l * b.nc + c;
-        M::template face_states<RECON>(b, D, n, N, l, u, s, ax, qL[l], qR[l]);
+      for (int l = 0; l < nv; ++l) {
+        if constexpr (D == 0)
+          M::template face_states<RECON>(b, D, n, N, l, lds_row + l * (FLUX_I_SPAN + 5), 1, ax, qL[l], qR[l]);
+        else M::template face_states<RECON>(b, D, n, N, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
       }
+    } else {
+#pragma unroll
+      for (int l = 0; l < nv; ++l)
+        M::template inner_states<RECON>(b, D, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
     }
     if (store_csnd) csf = T(0.5) * (tsqrt(T(b.gm) * qL[4] / qL[0]) + tsqrt(T(b.gm) * qR[4] / qR[0]));
     const T zero = T((n == 1) ? (double)b.mz[D][0] : (n == N) ? (double)b.mz[D][1] : 1.0);
