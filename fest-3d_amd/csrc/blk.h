@@ -45,9 +45,13 @@ struct Blk {
   double *src;                // SST source S_k, S_w (and lctm2015's S_gamma) of the interior cells (x volume)
   double *dvdy;               // lctm2015: the wall-normal sensor of each cell (k_lctm_sensor)
   // LU-SGS inputs and sweep values in hyperplane-major storage (k_lusgs.h)
-  int sk_j;                   // jmx + 1: positions per k row of a hyperplane
-  long sk_p, sk_n;            // positions per hyperplane; hyperplanes x sk_p
-  double *sk;                 // 3 nv + 23 components x sk_n
+  int sk_j, sk_g;             // positions per k row of a hyperplane; groups of 8 positions per hyperplane
+  double *sk;                 // 2 sk_npair(nv) values of every position
+  // sweep values handed between the tiles of columns of an LU-SGS sweep
+  // (k_lusgs_march): across the tile boundaries along j and along k
+  double *xj, *xk;
+  unsigned long long *ticket; // work-groups started by the sweeps so far
+  int lu_tj, lu_tk;           // columns of a tile along j and k (powers of two)
   double *g[3];
   // FP32 mode: FP32 copies of the padded state (refreshed after the ghost
   // cells of every residual evaluation) and of the gradients, read by the
@@ -86,7 +90,7 @@ struct Blk {
   double CFLv;                // CFL of the current call
 };
 
-enum : unsigned { ERR_NONPHYS = 1u, ERR_NAN_FLUX = 2u, ERR_NAN_GRAD = 4u, ERR_NAN_MU = 8u, ERR_CONFIG = 16u };
+enum : unsigned { ERR_NONPHYS = 1u, ERR_NAN_FLUX = 2u, ERR_NAN_GRAD = 4u, ERR_NAN_MU = 8u, ERR_CONFIG = 16u, ERR_SWEEP = 32u };
 
 __host__ __device__ inline long ci(const Blk &b, int i, int j, int k) {
   return (long)(i + 2) + (long)b.pi * ((long)(j + 2) + (long)b.pj * (long)(k + 2));
@@ -166,6 +170,22 @@ __device__ __forceinline__ double fmx(double a, double b) { return a > b ? a : b
 __device__ __forceinline__ double fmn(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ double fsgn(double a, double b) { return copysign(fabs(a), b); }
 __device__ __forceinline__ double sqd(double x) { return x * x; }
+// The compiler's FP64 quotient: v_rcp_f64, two Newton steps, the quotient and
+// its remainder correction -- wrapped in v_div_scale, v_div_fmas and
+// v_div_fixup, which rescale operands near the ends of the exponent range.
+// The wrapper costs 3 of 11 instructions and runs every quotient of a thread
+// through VCC one after the other.  qdiv is the same sequence without it: the
+// same bits wherever b, 1/b and the quotient are normal numbers, as they are
+// for the face arithmetic's quotients (|b| from 1e-28, the WENO weights, to
+// 1e64).  Not for quotients that may be 0/0 or x/0: those take NaN here
+// (bmuscl_cell divides by plain differences and keeps a / b).
+__device__ __forceinline__ double qdiv(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
 // FP32 forms for the single-precision face arithmetic
 __device__ __forceinline__ float fmx(float a, float b) { return a > b ? a : b; }
 __device__ __forceinline__ float fmn(float a, float b) { return a < b ? a : b; }

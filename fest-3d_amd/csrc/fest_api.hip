@@ -248,12 +248,26 @@ inline void box(long ni, long nj, long nk, dim3 &g, dim3 &t, int pad8 = 0) {
   g = dim3(plane_slots(cdiv(ni * nj, FLAT_BLOCK), pad8), (unsigned)nk, 1);
 }
 
+// doubles of the sweeps' hand-over slots across the tile boundaries along j and k
+long lu_slots_j(const Blk &b) { return (long)(cdiv(b.jmx - 1, b.lu_tj) - 1) * (b.kmx - 1) * (b.imx - 1) * LU_SLOT; }
+long lu_slots_k(const Blk &b) { return (long)(cdiv(b.kmx - 1, b.lu_tk) - 1) * (b.jmx - 1) * (b.imx - 1) * LU_SLOT; }
+void lu_empty_slots(fest_handle *h) {
+  const Blk &b = h->b;
+  const long nj = lu_slots_j(b), nk = lu_slots_k(b);
+  if (nj) hipLaunchKernelGGL(k_lusgs_empty, dim3(cdiv(nj, 256)), dim3(256), 0, h->stream, b.xj, nj);
+  if (nk) hipLaunchKernelGGL(k_lusgs_empty, dim3(cdiv(nk, 256)), dim3(256), 0, h->stream, b.xk, nk);
+}
+
 int check_err(fest_handle *h) {
   unsigned e = 0;
   HIPCHK(h, hipMemcpyAsync(&e, h->b.err, sizeof(unsigned), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if (!e) return 0;
   HIPCHK(h, hipMemsetAsync(h->b.err, 0, sizeof(unsigned), h->stream));
+  if (e & ERR_SWEEP) {
+    lu_empty_slots(h);
+    return fail(h, FEST_E_HIP, "an LU-SGS sweep's wait for a neighbouring tile ran out");
+  }
   if (e & ERR_NONPHYS) return fail(h, FEST_E_NONPHYSICAL, "non-physical state (rho<0, p<0 or NaN) in the update");
   if (e & ERR_NAN_FLUX) return fail(h, FEST_E_NAN, "NaN in the face fluxes");
   if (e & ERR_NAN_GRAD) return fail(h, FEST_E_NAN, "NaN in the gradients");
@@ -421,15 +435,14 @@ int launch_update(fest_handle *h, double TF, double SF, int flags) {
 }
 
 // LU-SGS update (src/lusgs.f90:134-183): the hyperplane-major copies and
-// the diagonal, one launch per hyperplane i + j + k = s forward and
-// backward, then qp += delQ
-// copies up to 8 planes into hyperplane-major components c0.. (k_to_skew)
-void to_skew(fest_handle *h, std::initializer_list<const double *> planes, int c0, int layout, int lo, int hi) {
+// the diagonal, one launch per sweep, then qp += delQ
+// copies up to 8 planes into hyperplane-major pairs p0.. (k_to_skew)
+void to_skew(fest_handle *h, std::initializer_list<const double *> planes, int p0, int layout, int lo, int hi) {
   Blk &b = h->b;
   SkewIn a{};
   a.n = 0;
   for (const double *p : planes) a.p[a.n++] = p;
-  a.c0 = c0;
+  a.p0 = p0;
   a.layout = layout;
   a.lo = lo;
   a.hi = hi;
@@ -438,7 +451,7 @@ void to_skew(fest_handle *h, std::initializer_list<const double *> planes, int c
   hipLaunchKernelGGL(k_to_skew, g, dim3(256), 0, h->stream, b, a);
 }
 
-template <int NV>
+template <int NV, bool KKL = false>
 int launch_lusgs_nv(fest_handle *h) {
   using C = Sk<NV>;
   Blk &b = h->b;
@@ -448,13 +461,11 @@ int launch_lusgs_nv(fest_handle *h) {
   {
     KgScope ts(h, KG_LU_DIAG);
     if (!h->sk_geometry) {
-      // volumes and faces: once per grid
-      to_skew(h, {b.vol}, C::VOL, 0, 0, 1);
-      for (int d = 0; d < 3; ++d) to_skew(h, {b.fA[d], b.fx[d], b.fy[d], b.fz[d]}, C::FACE + 4 * d, 2 + d, 1, 1);
+      // the faces: once per grid
+      for (int d = 0; d < 3; ++d) to_skew(h, {b.fA[d], b.fx[d], b.fy[d], b.fz[d]}, C::FACE + C::NF * d, 2 + d, 1, 1);
       h->sk_geometry = true;
     }
-    const long nc = b.nc, nr = b.nres;
-    // the NV state planes and residue planes (at most 7, one transpose each)
+    const long nc = b.nc;
     if (NV == 7)
       to_skew(h, {b.qp, b.qp + nc, b.qp + 2 * nc, b.qp + 3 * nc, b.qp + 4 * nc, b.qp + 5 * nc, b.qp + 6 * nc},
               C::Q, 0, 0, 1);
@@ -462,26 +473,16 @@ int launch_lusgs_nv(fest_handle *h) {
       to_skew(h, {b.qp, b.qp + nc, b.qp + 2 * nc, b.qp + 3 * nc, b.qp + 4 * nc, b.qp + 5 * nc}, C::Q, 0, 0, 1);
     else
       to_skew(h, {b.qp, b.qp + nc, b.qp + 2 * nc, b.qp + 3 * nc, b.qp + 4 * nc}, C::Q, 0, 0, 1);
-    to_skew(h, {b.mu, b.mut, b.f1}, C::MU, 0, 0, 1);
-    if (NV == 7)
-      to_skew(h, {b.res, b.res + nr, b.res + 2 * nr, b.res + 3 * nr, b.res + 4 * nr, b.res + 5 * nr, b.res + 6 * nr},
-              C::RES, 1, 1, 0);
-    else if (NV == 6)
-      to_skew(h, {b.res, b.res + nr, b.res + 2 * nr, b.res + 3 * nr, b.res + 4 * nr, b.res + 5 * nr}, C::RES, 1, 1, 0);
-    else
-      to_skew(h, {b.res, b.res + nr, b.res + 2 * nr, b.res + 3 * nr, b.res + 4 * nr}, C::RES, 1, 1, 0);
     // radii, Old fluxes and diagonal over the cells 1..n+1
     const dim3 gp((unsigned)(cdiv(b.imx, 16) * cdiv(b.jmx, 16)), (unsigned)b.kmx);
-    hipLaunchKernelGGL(k_lusgs_prep<NV>, gp, dim3(256), 0, st, b);
+    hipLaunchKernelGGL((k_lusgs_prep<NV, KKL>), gp, dim3(256), 0, st, b);
   }
   LAUNCHCHK(h);
-  const int smax = (b.imx - 1) + (b.jmx - 1) + (b.kmx - 1);
-  // four lanes per (j, k) pair
-  const dim3 gs(cdiv(4L * (b.jmx - 1) * (b.kmx - 1), 256)), ts256(256);
+  const dim3 gs(cdiv(b.jmx - 1, b.lu_tj) * cdiv(b.kmx - 1, b.lu_tk)), ts(4 * LU_COLUMNS);
   {
-    KgScope ts(h, KG_LU_SWEEP);
-    for (int s = 3; s <= smax; ++s) hipLaunchKernelGGL((k_lusgs_sweep<NV, 0>), gs, ts256, 0, st, b, s);
-    for (int s = smax; s >= 3; --s) hipLaunchKernelGGL((k_lusgs_sweep<NV, 1>), gs, ts256, 0, st, b, s);
+    KgScope sc(h, KG_LU_SWEEP);
+    hipLaunchKernelGGL((k_lusgs_march<NV, 0, KKL>), gs, ts, 0, st, b);
+    hipLaunchKernelGGL((k_lusgs_march<NV, 1, KKL>), gs, ts, 0, st, b);
   }
   LAUNCHCHK(h);
   {
@@ -492,6 +493,7 @@ int launch_lusgs_nv(fest_handle *h) {
   return 0;
 }
 int launch_lusgs(fest_handle *h) {
+  if (h->b.kkl) return launch_lusgs_nv<7, true>(h);
   return h->b.nv == 7 ? launch_lusgs_nv<7>(h) : h->b.nv == 6 ? launch_lusgs_nv<6>(h) : launch_lusgs_nv<5>(h);
 }
 
@@ -883,12 +885,21 @@ int fest_create(fest_handle **out, const fest_extent *dims, const fest_scheme *s
   if (b.time_acc == FEST_TA_IMPLICIT) {
     // LU-SGS storage over the hyperplanes of (0:imx, 0:jmx, 0:kmx); zero
     // where nothing is written (the sweep values outside the interior)
-    b.sk_j = b.jmx + 1;
-    b.sk_p = (long)b.sk_j * (b.kmx + 1);
-    b.sk_n = (long)(b.imx + b.jmx + b.kmx + 1) * b.sk_p;
-    const long nsk = sk_ncomp(b.nv) * b.sk_n;
+    b.sk_j = (b.jmx + 15) / 8 * 8;  // j = 0..jmx at 7..jmx+7
+    b.sk_g = b.sk_j / 8 * (b.kmx + 1);
+    const long nsk = (long)sk_npair(b.nv) * 16 * b.sk_g * (b.imx + b.jmx + b.kmx + 1);
     AL(b.sk, nsk);
     HIPCHK(h, hipMemsetAsync(b.sk, 0, sizeof(double) * nsk, h->stream));
+    // tiles of 64 columns, square unless the block is thin in k
+    b.lu_tk = 1;
+    while (b.lu_tk < 8 && b.lu_tk < b.kmx - 1) b.lu_tk *= 2;
+    b.lu_tj = LU_COLUMNS / b.lu_tk;
+    AL(b.xj, lu_slots_j(b)); AL(b.xk, lu_slots_k(b));
+    double *tk = nullptr;
+    AL(tk, 1);
+    b.ticket = (unsigned long long *)tk;
+    HIPCHK(h, hipMemsetAsync(tk, 0, sizeof(double), h->stream));
+    lu_empty_slots(h);
   }
 #undef AL
   void *e = nullptr;

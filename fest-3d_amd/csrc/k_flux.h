@@ -29,22 +29,6 @@
 
 namespace fest {
 
-// The compiler's FP64 quotient: v_rcp_f64, two Newton steps, the quotient and
-// its remainder correction -- wrapped in v_div_scale, v_div_fmas and
-// v_div_fixup, which rescale operands near the ends of the exponent range.
-// The wrapper costs 3 of 11 instructions and runs every quotient of a thread
-// through VCC one after the other.  qdiv is the same sequence without it: the
-// same bits wherever b, 1/b and the quotient are normal numbers, as they are
-// for the face arithmetic's quotients (|b| from 1e-28, the WENO weights, to
-// 1e64).  Not for quotients that may be 0/0 or x/0: those take NaN here
-// (bmuscl_cell divides by plain differences and keeps a / b).
-__device__ __forceinline__ double qdiv(double a, double b) {
-  double y = __builtin_amdgcn_rcp(b);
-  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
-  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
-  const double q = a * y;
-  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
-}
 // FP64: correctly rounded.  FP32 (the mixed-precision mode): the
 // hardware reciprocal and square root (v_rcp_f32, v_sqrt_f32, 1 ulp), whose
 // error is far below the FP32 face arithmetic's own.

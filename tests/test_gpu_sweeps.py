@@ -48,3 +48,26 @@ def test_boundary_and_inner_faces(ni, nj, nk, recon):
     out = g.download("qp", "F", "G", "H", "residue")
     for n, on in (("qp", "qp"), ("F", "F"), ("G", "G"), ("H", "H"), ("residue", "res")):
         assert relerr(out[n], o.arr(on)) <= TOL, n
+
+
+@pytest.mark.parametrize("turb", ["none", "sst", "sa", "kkl"])
+@pytest.mark.parametrize("ni,nj,nk", [(5, 70, 1), (4, 64, 1), (6, 7, 3), (5, 17, 4), (7, 9, 8), (3, 17, 9), (9, 8, 16)])
+def test_implicit_sweep_tiles(ni, nj, nk, turb):
+    """LU-SGS sweeps where their 64-column tiles (64 x 1, 16 x 4 or 8 x 8) are
+    full, just exceeded or mostly empty: one tile, a chain along j, both
+    directions.  Two steps, every one handing values over the tile edges."""
+    if turb == "none":
+        case, nodes, q = C.laminar_box(ni, nj, nk)
+        case = dataclasses.replace(case, time_local=1, bc_id=(-8, -4, -5, -6, -6, -6), fix_p=(case.p_inf,) * 6)
+        nodes = C.cartesian_nodes(case, warp=0.03)
+    else:
+        case, nodes, q = C.sst_bump(ni, nj, nk, turb=turb, recon="muscl", first=2e-3)
+        case = dataclasses.replace(case, bc_id=case.bc_id[:4] + (-6, -6))
+    case = dataclasses.replace(case, time_accuracy="implicit")
+    print("tiles", ni, nj, nk, turb, flush=True)
+    g, o = pair(case, nodes, q, turb != "none")
+    for it in (1, 2):
+        assert o.step(it) == 0
+        g.get_next_solution(it)
+    inner = (slice(None),) + (slice(3, -3),) * 3
+    assert relerr(g.download("qp")[inner], o.arr("qp")[inner]) <= TOL
