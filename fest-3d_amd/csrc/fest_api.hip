@@ -104,8 +104,8 @@ struct fest_handle {
 // itself and leaves the group unusable (its links point into the block)
 // the phases of a batched group step (k_multi.h), each one launch over the
 // tiles of every block
-enum { PH_BEGIN = 0, PH_BC_A0, PH_BC_A1, PH_BC_A2, PH_BC_B0, PH_BC_B1, PH_BC_B2, PH_EDGE0, PH_EDGE1, PH_EDGE2,
-       PH_F32, PH_GRAD, PH_GRAD_BC, PH_FLUX_I, PH_FLUX_J, PH_FLUX_K, PH_DT, PH_UPDATE, PH_COUNT };
+enum { PH_BEGIN = 0, PH_BC0, PH_BC1, PH_BC2, PH_BC3, PH_BC4, PH_BC5, PH_EDGES, PH_F32, PH_GRAD, PH_GRAD_BC,
+       PH_FLUX_I, PH_FLUX_J, PH_FLUX_K, PH_DT, PH_UPDATE, PH_COUNT };
 
 struct fest_group {
   std::vector<fest_handle *> blocks;
@@ -281,36 +281,61 @@ inline void tiles(long ni, long nj, long nk, dim3 &g, dim3 &t, int pad8) {
   g = dim3(plane_slots((long)cdiv(ni, TILE_I) * cdiv(nj, TILE_J), pad8), (unsigned)nk, 1);
 }
 
-// C2: the ghost cells of the block's own boundary rules, face by face, then
-// the edges and corners
+// The launches of a block's faces, in the reference's order imin, imax, jmin,
+// ...: the first and the last face of each.  Faces share a launch when none
+// reads what another writes.  A direction's two faces read its interior
+// layers 1..4 only if it has at least 4 cells.  Consecutive directions are
+// taken together, but not one with a periodic face, whose plane copy reads the
+// other directions' ghost cells (those before it filled, those after it not
+// yet), nor two with a far field or total-pressure inlet, whose plane copies
+// meet at the edges.
+std::vector<std::pair<int, int>> bc_launches(const Blk &b) {
+  std::vector<std::pair<int, int>> v;
+  bool open = false, planes = false;  // the last launch may take more; it holds plane copies
+  for (int d = 0; d < 3; ++d) {
+    const int N = d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx, lo = b.bc[2 * d], hi = b.bc[2 * d + 1];
+    const bool plane = lo == -8 || hi == -8 || lo == -11 || hi == -11;
+    if (N < 5) {
+      v.push_back({2 * d, 2 * d});
+      v.push_back({2 * d + 1, 2 * d + 1});
+      open = false;
+    } else if (lo == -9 || hi == -9) {
+      v.push_back({2 * d, 2 * d + 1});
+      open = false;
+    } else if (open && !(plane && planes)) {
+      v.back().second = 2 * d + 1;
+      planes |= plane;
+    } else {
+      v.push_back({2 * d, 2 * d + 1});
+      open = true;
+      planes = plane;
+    }
+  }
+  return v;
+}
+// tiles of 64 x 4 columns over the padded plane of a face
+dim3 bc_grid(const Blk &b, int face) { return dim3(cdiv(face_na(b, face) + 5, 64), cdiv(face_nb(b, face) + 5, 4), 1); }
+
+// C2: the ghost cells of the block's own boundary rules, then the edges and
+// corners
 int launch_ghosts(fest_handle *h, int current_iter) {
   Blk &b = h->b;
   hipStream_t st = h->stream;
-  // faces in the reference's order imin, imax, jmin, ...; the two faces of
-  // one direction share a launch when the direction has at least 8 nodes:
-  // each side then reads only its own interior layers 1..4 and ghost layers,
-  // so neither sees the other's writes
   {
-  KgScope ts(h, KG_BC_FACE);
-  for (int d = 0; d < 3; ++d) {
-    int N = d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx;
-    int na = face_na(b, 2 * d), nb = face_nb(b, 2 * d);
-    dim3 t(64, 4, 1);
-    if (N >= 8) {
-      dim3 g(cdiv(na + 5, 64), cdiv(nb + 5, 4), 2);
-      hipLaunchKernelGGL(k_bc_face, g, t, 0, st, b, 2 * d, current_iter);
-    } else {
-      dim3 g(cdiv(na + 5, 64), cdiv(nb + 5, 4), 1);
-      hipLaunchKernelGGL(k_bc_face, g, t, 0, st, b, 2 * d, current_iter);
-      hipLaunchKernelGGL(k_bc_face, g, t, 0, st, b, 2 * d + 1, current_iter);
+    KgScope ts(h, KG_BC_FACE);
+    for (auto &f : bc_launches(b)) {
+      dim3 g(1, 1, (unsigned)(f.second - f.first + 1));
+      for (int face = f.first; face <= f.second; ++face) {
+        const dim3 one = bc_grid(b, face);
+        g.x = std::max(g.x, one.x);
+        g.y = std::max(g.y, one.y);
+      }
+      hipLaunchKernelGGL(k_bc_face, g, dim3(64, 4, 1), 0, st, b, f.first, current_iter);
     }
-  }
   }
   {
     KgScope ts(h, KG_BC_EDGES);
-    hipLaunchKernelGGL(k_bc_edges, dim3(cdiv(4L * (b.imx + 5) * b.nv, 256)), dim3(256), 0, st, b, 0);
-    hipLaunchKernelGGL(k_bc_edges, dim3(cdiv(4L * (b.kmx + 5) * b.nv, 256)), dim3(256), 0, st, b, 1);
-    hipLaunchKernelGGL(k_bc_edges, dim3(1), dim3(64), 0, st, b, 2);
+    hipLaunchKernelGGL(k_bc_edges, dim3(cdiv(edge_cells(b) * b.nv, 256)), dim3(256), 0, st, b);
   }
   LAUNCHCHK(h);
   return 0;
@@ -1375,22 +1400,9 @@ int group_exchange(fest_group *g) {
 // step operations lay it out); false when the block has no tiles in it
 bool phase_grid(const Blk &b, int ph, dim3 &g, int ti = TILE_I) {
   const int tj = 256 / ti;
-  auto N = [&](int d) { return d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx; };
   switch (ph) {
     case PH_BEGIN: g = dim3(cdiv(b.nc, 256), 1, 1); return true;
-    case PH_BC_A0: case PH_BC_A1: case PH_BC_A2: {
-      const int d = ph - PH_BC_A0;
-      g = dim3(cdiv(face_na(b, 2 * d) + 5, 64), cdiv(face_nb(b, 2 * d) + 5, 4), N(d) >= 8 ? 2 : 1);
-      return true;
-    }
-    case PH_BC_B0: case PH_BC_B1: case PH_BC_B2: {
-      const int d = ph - PH_BC_B0;
-      g = dim3(cdiv(face_na(b, 2 * d) + 5, 64), cdiv(face_nb(b, 2 * d) + 5, 4), 1);
-      return N(d) < 8;
-    }
-    case PH_EDGE0: g = dim3(cdiv(4L * (b.imx + 5) * b.nv, 256), 1, 1); return true;
-    case PH_EDGE1: g = dim3(cdiv(4L * (b.kmx + 5) * b.nv, 256), 1, 1); return true;
-    case PH_EDGE2: g = dim3(1, 1, 1); return true;
+    case PH_EDGES: g = dim3(cdiv(edge_cells(b) * b.nv, 256), 1, 1); return true;
     case PH_F32: g = dim3(cdiv(b.nc * b.nv, 256), 1, 1); return b.fp32 != 0;
     case PH_GRAD: g = dim3(cdiv((long)(b.imx + 1) * (b.jmx + 1), FLAT_BLOCK), b.kmx + 1, 1); return b.mu_ref != 0.0;
     case PH_GRAD_BC: {
@@ -1437,6 +1449,19 @@ int build_lists(fest_group *g, int order) {
     for (size_t n = 0; n < g->blocks.size(); ++n) {
       const Blk &b = g->blocks[n]->b;
       dim3 gr;
+      if (ph >= PH_BC0 && ph <= PH_BC5) {
+        // the block's launch of this number, exact tiles of each face; none
+        // on interface faces
+        const auto launches = bc_launches(b);
+        if (ph - PH_BC0 >= (int)launches.size()) continue;
+        for (int z = launches[ph - PH_BC0].first; z <= launches[ph - PH_BC0].second; ++z) {
+          if (b.bc[z] >= 0 || b.bc[z] == -10) continue;
+          const dim3 f = bc_grid(b, z);
+          for (unsigned y = 0; y < f.y; ++y)
+            for (unsigned x = 0; x < f.x; ++x) per[n].push_back(WorkItem{(int)n, (int)x, (int)y, z});
+        }
+        continue;
+      }
       if (!phase_grid(b, ph, gr, g->tile_i)) continue;
       if (ph == PH_GRAD_BC) {
         // the ghost-gradient rule per face, exact tiles of the face
@@ -1513,13 +1538,8 @@ int run_group_op_batched(fest_group *g, const StepOp &op, int current_iter) {
     case OP_BEGIN: KM(PH_BEGIN, km_step_begin, dim3(256), op.flags); break;
     case OP_RESID:
       if ((rc = group_exchange(g))) return rc;
-      for (int d = 0; d < 3; ++d) {
-        KM(PH_BC_A0 + d, km_bc_face, dim3(64, 4, 1), 2 * d, current_iter);
-        KM(PH_BC_B0 + d, km_bc_face, dim3(64, 4, 1), 2 * d + 1, current_iter);
-      }
-      KM(PH_EDGE0, km_bc_edges, dim3(256), 0);
-      KM(PH_EDGE1, km_bc_edges, dim3(256), 1);
-      KM(PH_EDGE2, km_bc_edges, dim3(256), 2);
+      for (int ph = PH_BC0; ph <= PH_BC5; ++ph) KM(ph, km_bc_face, dim3(64, 4, 1), current_iter);
+      KM(PH_EDGES, km_bc_edges, dim3(256));
       if (b0.fp32) KM(PH_F32, km_to_f32, dim3(256));
       if (b0.mu_ref != 0.0) {
         if (b0.g32only) {

@@ -51,46 +51,7 @@ __device__ __forceinline__ FaceBC face_params(const Blk &b, int face) {
   return p;
 }
 
-// src/boundary/copy_bc.f90:58-131 on one column
-__device__ __forceinline__ void copy3col(const Blk &b, double *v, int type, int face, int a, int bb) {
-  double a1, a2, a3;
-  if (type == CP_ANTI) { a1 = 1.; a2 = -1.; a3 = 0.; }
-  else if (type == CP_FLAT) { a1 = 1.; a2 = 1.; a3 = 0.; }
-  else { a1 = b.c1; a2 = b.c2; a3 = b.c3; }
-  // ghost layer g takes interior layer g+1 (anti, symm) or layer 1 (flat)
-#pragma unroll
-  for (int g = 0; g < 3; ++g) {
-    const int src = type == CP_FLAT ? 1 : g + 1;
-    v[fcell(b, face, -g, a, bb)] = (a2 * v[fcell(b, face, src, a, bb)] - a3 * v[fcell(b, face, src + 1, a, bb)]) / a1;
-  }
-}
-
-// src/boundary/bc_primitive.f90:484-525 on one column
-__device__ __forceinline__ void fixcol(const Blk &b, double *v, double val, int face, int a, int bb) {
-#pragma unroll
-  for (int g = 0; g < 3; ++g) v[fcell(b, face, -g, a, bb)] = val;
-}
-
-// the turbulence variables: k and omega (SST), k and kL (k-kL), nu-tilde
-// (SA); lctm2015's intermittency takes a flat copy wherever they copy
-// (bc_primitive.f90:302, 385, 437, 475, 555) and its own fixed value
-// wherever they are fixed (:262, :343).  kl_tw: the subsonic inlet fixes
-// k-kL's kL from the omega values (src/boundary/bc_primitive.f90:333-336),
-// which k-kL never reads from the boundary file (read_bc.f90:98-108)
 __device__ __forceinline__ bool two_eq(const Blk &b) { return b.ng >= 6; }
-__device__ __forceinline__ void turb_copycol(const Blk &b, int type, int face, int a, int bb) {
-  if (b.ng >= 5) copy3col(b, b.qp + 5 * b.nc, type, face, a, bb);
-  if (two_eq(b)) copy3col(b, b.qp + 6 * b.nc, type, face, a, bb);
-  if (b.lctm) copy3col(b, b.qp + 7 * b.nc, CP_FLAT, face, a, bb);
-}
-__device__ __forceinline__ void turb_fixcol(const Blk &b, const FaceBC &p, int face, int a, int bb, bool kl_tw = false) {
-  if (two_eq(b)) {
-    fixcol(b, b.qp + 5 * b.nc, p.fix[FX_TK], face, a, bb);
-    fixcol(b, b.qp + 6 * b.nc, (b.kkl && !kl_tw) ? p.fix[FX_TKL] : p.fix[FX_TW], face, a, bb);
-  }
-  if (b.ng == 5) fixcol(b, b.qp + 5 * b.nc, p.fix[FX_TV], face, a, bb);
-  if (b.lctm) fixcol(b, b.qp + 7 * b.nc, p.fix[FX_TGM], face, a, bb);
-}
 
 // unit normal of the boundary face at (a, bb); the metric planes are picked
 // per case with constant member indices (a run-time index into the
@@ -107,40 +68,6 @@ __device__ __forceinline__ void bnormal(const Blk &b, int face, int a, int bb, d
     default: f = fi(b, 2, a, bb, b.kmx); px = b.fx[2]; py = b.fy[2]; pz = b.fz[2]; break;
   }
   nx = px[f]; ny = py[f]; nz = pz[f];
-}
-
-// src/boundary/bc_primitive.f90:1778-1945
-__device__ __forceinline__ void temp_based_density_col(const Blk &b, const FaceBC &p_, int face, int a, int bb) {
-  double Tw = p_.fix[FX_TWALL], R = b.R, gm = b.gm;
-  double *rho = b.qp, *p = b.qp + 4 * b.nc;
-  if (Tw < 0.0) {
-    long c1 = fcell(b, face, 1, a, bb);
-    double stag = (p[c1] / (R * rho[c1])) * (1 + (0.5 * (gm - 1.) * gm * p[c1] / rho[c1]));
-    for (int g = 0; g < 3; ++g) {
-      long cg = fcell(b, face, -g, a, bb);
-      rho[cg] = p[cg] / (R * stag);
-    }
-  } else if (Tw > 1.0) {
-    for (int g = 0; g < 3; ++g) {
-      long cg = fcell(b, face, -g, a, bb), cn = fcell(b, face, 1 + g, a, bb);
-      rho[cg] = p[cg] / (R * (2 * Tw - (p[cn] / (R * rho[cn]))));
-    }
-  } else {
-    copy3col(b, rho, CP_SYMM, face, a, bb);
-  }
-}
-
-// src/boundary/bc_primitive.f90:564-643 (Sutherland mu whatever mu_variation)
-__device__ __forceinline__ void omega_wall_col(const Blk &b, int face, int a, int bb) {
-  double *rho = b.qp, *p = b.qp + 4 * b.nc, *tw = b.qp + 6 * b.nc;
-  long c0 = fcell(b, face, 0, a, bb), c1 = fcell(b, face, 1, a, bb);
-  for (int l = 1; l <= 3; ++l) {
-    double T_face = 0.5 * ((p[c0] / rho[c0]) + (p[c1] / rho[c1])) / b.R;
-    double mu = b.mu_ref * pow(T_face / b.T_ref, 1.5) * ((b.T_ref + b.S_ref) / (T_face + b.S_ref));
-    double r = 0.5 * (rho[c0] + rho[c1]);
-    double d2 = 2 * b.dist[c1];
-    tw[fcell(b, face, 1 - l, a, bb)] = 120 * mu / (r * 0.075 * (d2 * d2)) - tw[fcell(b, face, l, a, bb)];
-  }
 }
 
 // far-field Riemann state of one column (src/boundary/bc_primitive.f90:645-1234)
@@ -194,209 +121,295 @@ __device__ __forceinline__ T riemann_state(const Blk &b, int face, const T (&c)[
   }
   return Unb;
 }
-// riemann_state on the resident state; when write != 0 it stores layer 0
-// of rho, u, v, w, p
-__device__ __forceinline__ double riemann_col(const Blk &b, int face, int a, int bb, int write, bool total, double tp) {
-  const long c1 = fcell(b, face, 1, a, bb), cg = fcell(b, face, 0, a, bb);
+// Unb of the far-field or total-pressure state at column (a, bb)
+__device__ __forceinline__ double riemann_unb(const Blk &b, int face, int a, int bb) {
+  const long c1 = fcell(b, face, 1, a, bb);
   double c[5], g[5], nrm[3];
 #pragma unroll
   for (int l = 0; l < 5; ++l) c[l] = b.qp[(long)l * b.nc + c1];
   bnormal(b, face, a, bb, nrm[0], nrm[1], nrm[2]);
-  const double Unb = riemann_state(b, face, c, nrm, write != 0, total, tp, g);
-  if (write) {
-#pragma unroll
-    for (int l = 0; l < 5; ++l) b.qp[(long)l * b.nc + cg] = g[l];
-  }
-  return Unb;
+  return riemann_state(b, face, c, nrm, false, false, 0.0, g);
 }
 
-// src/boundary/FT_bc.f90:36-106; j and k faces reflect with the I-face
-// normal stored at the same index, as the reference does
-__device__ __forceinline__ void flow_tangency_col(const Blk &b, int face, int a, int bb) {
-  double *u = b.qp + b.nc, *v = b.qp + 2 * b.nc, *w = b.qp + 3 * b.nc;
-  double nx, ny, nz;
-  bnormal(b, face, a, bb, nx, ny, nz);
-  long f;
-  switch (face) {
-    case 0: f = fi(b, 0, 1, a, bb); break;
-    case 1: f = fi(b, 0, b.imx, a, bb); break;
-    case 2: f = fi(b, 0, a, 1, bb); break;
-    case 3: f = fi(b, 0, a, b.jmx, bb); break;
-    case 4: f = fi(b, 0, a, bb, 1); break;
-    default: f = fi(b, 0, a, bb, b.kmx); break;
-  }
-  double rx = b.fx[0][f], ry = b.fy[0][f], rz = b.fz[0][f];
-  for (int l = 1; l <= 3; ++l) {
-    long c = fcell(b, face, l, a, bb), g = fcell(b, face, 1 - l, a, bb);
-    double dot = u[c] * nx + v[c] * ny + w[c] * nz;
-    u[g] = u[c] - (2.0 * dot * rx);
-    v[g] = v[c] - (2.0 * dot * ry);
-    w[g] = w[c] - (2.0 * dot * rz);
-  }
+// How a variable's three ghost cells follow from its first four interior
+// cells (src/boundary/copy_bc.f90:58-131, bc_primitive.f90:484-525), or not:
+// left as they are
+enum { BK_LEFT = -1, BK_ANTI = CP_ANTI, BK_FLAT = CP_FLAT, BK_SYMM = CP_SYMM, BK_FIX = 3 };
+constexpr int BC_NV = 8;
+
+// The rules of every variable of a face: the turbulence variables are k and
+// omega (SST), k and kL (k-kL), nu-tilde (SA); lctm2015's intermittency takes
+// a flat copy wherever they copy (bc_primitive.f90:302, 385, 437, 475, 555) and
+// its own fixed value wherever they are fixed (:262, :343).  kl_tw: the
+// subsonic inlet fixes k-kL's kL from the omega values
+// (src/boundary/bc_primitive.f90:333-336), which k-kL never reads from the
+// boundary file (read_bc.f90:98-108)
+struct BcRules {
+  int kind[BC_NV];
+  double val[BC_NV];
+};
+__device__ __forceinline__ void turb_copy(const Blk &b, BcRules &r, int kind) {
+  if (b.ng >= 5) r.kind[5] = kind;
+  if (two_eq(b)) r.kind[6] = kind;
+  if (b.lctm) r.kind[7] = BK_FLAT;
+}
+__device__ __forceinline__ void turb_fix(const Blk &b, const FaceBC &p, BcRules &r, bool kl_tw) {
+  if (b.ng >= 5) r.kind[5] = BK_FIX;
+  r.val[5] = two_eq(b) ? p.fix[FX_TK] : p.fix[FX_TV];
+  if (two_eq(b)) r.kind[6] = BK_FIX;
+  r.val[6] = (b.kkl && !kl_tw) ? p.fix[FX_TKL] : p.fix[FX_TW];
+  if (b.lctm) r.kind[7] = BK_FIX;
+  r.val[7] = p.fix[FX_TGM];
 }
 
-// One face of populate_ghost_primitive.  The grid spans the padded
+// One column of populate_ghost_primitive.  The grid spans the padded
 // tangential plane (-2..na+2) x (-2..nb+2); most conditions act on the face
 // interior 1..na-1 x 1..nb-1, the periodic and far-field plane copies on the
-// whole plane.
-// blockIdx.z selects face0 + z: the min and max faces of one direction run
-// in one launch when they cannot touch each other's cells (see the caller).
-__device__ __forceinline__ void k_bc_face_b(const Blk &b, const Wg &wg, int face0, int current_iter) {
-  const int face = face0 + (int)wg.z;
-  int a = (int)(wg.x * blockDim.x + threadIdx.x) - 2;
-  int bb = (int)(wg.y * blockDim.y + threadIdx.y) - 2;
-  int na = face_na(b, face), nb = face_nb(b, face);
+// whole plane.  A launch may hold several faces when none reads what another
+// writes (see the caller).  All of a column's cells are read before any is
+// written: a rule that reads and writes variable by variable waits for memory
+// once per variable.  With the launches joined (bc_launches) and the edges in
+// one, a stage's ghosts of the SST bump at 97x61x45 take 26 us, not 56, those
+// of the laminar box at 64x64x4 28, not 49.
+__device__ __forceinline__ void k_bc_face_b(const Blk &b, int face, int a, int bb, int current_iter) {
+  const int na = face_na(b, face), nb = face_nb(b, face);
   if (a > na + 2 || bb > nb + 2) return;
   const FaceBC p = face_params(b, face);
   const int id = p.id;
-  bool inner = (a >= 1 && a <= na - 1 && bb >= 1 && bb <= nb - 1);
-  double *q = b.qp;
+  if (id >= 0 || id == -10) return;  // filled by the interface exchange
+  const bool inner = a >= 1 && a <= na - 1 && bb >= 1 && bb <= nb - 1;
+  const bool riemann = id == -8 || id == -11;
+  double *const q = b.qp;
   const long nc = b.nc;
+  if (id == -9) {  // single-block periodic: whole plane, three layers
+    // the reference's array assignment reads its source layers whole
+    // before writing; with one or two cells in the direction they overlap
+    // the destination layers.  Layers g = 0..2 sit at d0 + g*st (ghosts)
+    // and s0 + g*st (their sources) along the face normal's stride st.
+    long d0, s0, st;
+    switch (face) {
+      case 0: d0 = ci(b, -2, a, bb); s0 = ci(b, b.imx - 3, a, bb); st = 1; break;
+      case 1: d0 = ci(b, b.imx, a, bb); s0 = ci(b, 1, a, bb); st = 1; break;
+      case 2: d0 = ci(b, a, -2, bb); s0 = ci(b, a, b.jmx - 3, bb); st = b.pi; break;
+      case 3: d0 = ci(b, a, b.jmx, bb); s0 = ci(b, a, 1, bb); st = b.pi; break;
+      case 4: d0 = ci(b, a, bb, -2); s0 = ci(b, a, bb, b.kmx - 3); st = (long)b.pi * b.pj; break;
+      default: d0 = ci(b, a, bb, b.kmx); s0 = ci(b, a, bb, 1); st = (long)b.pi * b.pj; break;
+    }
+    double v[BC_NV][3];
+#pragma unroll
+    for (int l = 0; l < BC_NV; ++l)
+      if (l < b.nv) {
+#pragma unroll
+        for (int g = 0; g < 3; ++g) v[l][g] = q[l * nc + s0 + g * st];
+      }
+#pragma unroll
+    for (int l = 0; l < BC_NV; ++l)
+      if (l < b.nv) {
+#pragma unroll
+        for (int g = 0; g < 3; ++g) q[l * nc + d0 + g * st] = v[l][g];
+      }
+    return;
+  }
+  if (!inner) {
+    // the far field's outer layers copy the first over the whole plane
+    if (!riemann) return;
+    const long g0 = fcell(b, face, 0, a, bb), g1 = fcell(b, face, -1, a, bb), g2 = fcell(b, face, -2, a, bb);
+    double v[BC_NV];
+#pragma unroll
+    for (int l = 0; l < BC_NV; ++l)
+      if (l < b.nv) v[l] = q[l * nc + g0];
+#pragma unroll
+    for (int l = 0; l < BC_NV; ++l)
+      if (l < b.nv) {
+        q[l * nc + g1] = v[l];
+        q[l * nc + g2] = v[l];
+      }
+    return;
+  }
+  // the rule of every variable
+  BcRules r;
+#pragma unroll
+  for (int l = 0; l < BC_NV; ++l) {
+    r.kind[l] = BK_LEFT;
+    r.val[l] = l < 5 ? p.fix[l] : 0.0;
+  }
+  auto flow = [&](int k0, int k1, int k2, int k3, int k4) {
+    r.kind[0] = k0; r.kind[1] = k1; r.kind[2] = k2; r.kind[3] = k3; r.kind[4] = k4;
+  };
+  const bool fix = current_iter <= 2;
   switch (id) {
     case -1:  // supersonic inlet
-      if (inner && current_iter <= 2) {
-        for (int l = 0; l < 5; ++l) fixcol(b, q + l * nc, p.fix[l], face, a, bb);
-        turb_fixcol(b, p, face, a, bb);
-      }
+      if (!fix) return;
+      flow(BK_FIX, BK_FIX, BK_FIX, BK_FIX, BK_FIX);
+      turb_fix(b, p, r, false);
       break;
     case -2:  // supersonic outlet
-      if (inner) {
-        for (int l = 0; l < 5; ++l) copy3col(b, q + l * nc, CP_FLAT, face, a, bb);
-        turb_copycol(b, CP_FLAT, face, a, bb);
-      }
+    case -7:  // pole
+      flow(BK_FLAT, BK_FLAT, BK_FLAT, BK_FLAT, BK_FLAT);
+      turb_copy(b, r, BK_FLAT);
       break;
     case -3:  // subsonic inlet
-      if (inner) {
-        if (current_iter <= 2) {
-          for (int l = 0; l < 4; ++l) fixcol(b, q + l * nc, p.fix[l], face, a, bb);
-          turb_fixcol(b, p, face, a, bb, true);
-        }
-        copy3col(b, q + 4 * nc, CP_FLAT, face, a, bb);
+      if (fix) {
+        flow(BK_FIX, BK_FIX, BK_FIX, BK_FIX, BK_LEFT);
+        turb_fix(b, p, r, true);
       }
+      r.kind[4] = BK_FLAT;
       break;
     case -4:  // subsonic outlet
-      if (inner) {
-        for (int l = 0; l < 4; ++l) copy3col(b, q + l * nc, CP_FLAT, face, a, bb);
-        if (current_iter <= 2) fixcol(b, q + 4 * nc, p.fix[FX_P], face, a, bb);
-        turb_copycol(b, CP_FLAT, face, a, bb);
+      flow(BK_FLAT, BK_FLAT, BK_FLAT, BK_FLAT, fix ? BK_FIX : BK_LEFT);
+      turb_copy(b, r, BK_FLAT);
+      break;
+    case -5:  // no-slip wall; the density by the wall temperature, SST's omega below
+      flow(BK_SYMM, BK_ANTI, BK_ANTI, BK_ANTI, BK_SYMM);
+      turb_copy(b, r, BK_ANTI);
+      if (two_eq(b) && !b.kkl) r.kind[6] = BK_LEFT;
+      break;
+    case -6:  // slip wall; the velocity below
+      flow(BK_SYMM, BK_LEFT, BK_LEFT, BK_LEFT, BK_SYMM);
+      turb_copy(b, r, BK_SYMM);
+      break;
+    case -8:   // far field
+    case -11:  // total-pressure inlet
+      // the whole-face turbulent copy/fix of the reference ends as set by
+      // the last face cell in its loop order
+      if (b.turb) {
+        if (riemann_unb(b, face, na - 1, nb - 1) > 0.) turb_copy(b, r, BK_FLAT);
+        else turb_fix(b, p, r, false);
       }
       break;
-    case -5:  // no-slip wall
-      if (inner) {
-        copy3col(b, q + 4 * nc, CP_SYMM, face, a, bb);
-        temp_based_density_col(b, p, face, a, bb);
-        copy3col(b, q + 1 * nc, CP_ANTI, face, a, bb);
-        copy3col(b, q + 2 * nc, CP_ANTI, face, a, bb);
-        copy3col(b, q + 3 * nc, CP_ANTI, face, a, bb);
-        if (b.ng >= 5) copy3col(b, q + 5 * nc, CP_ANTI, face, a, bb);  // k or nu-tilde
-        if (two_eq(b) && b.kkl) copy3col(b, q + 6 * nc, CP_ANTI, face, a, bb);  // kL, :548-550
-        else if (two_eq(b)) omega_wall_col(b, face, a, bb);
-        if (b.lctm) copy3col(b, q + 7 * nc, CP_FLAT, face, a, bb);  // :553-558
-      }
-      break;
-    case -6:  // slip wall
-      if (inner) {
-        copy3col(b, q, CP_SYMM, face, a, bb);
-        copy3col(b, q + 4 * nc, CP_SYMM, face, a, bb);
-        turb_copycol(b, CP_SYMM, face, a, bb);
-        flow_tangency_col(b, face, a, bb);
-      }
-      break;
-    case -7:  // pole
-      if (inner) {
-        for (int l = 0; l < 5; ++l) copy3col(b, q + l * nc, CP_FLAT, face, a, bb);
-        turb_copycol(b, CP_FLAT, face, a, bb);
-      }
-      break;
-    case -8:     // far field
-    case -11: {  // total-pressure inlet
-      const bool total = id == -11;
-      const double tp = p.fix[FX_TP];
-      if (inner) {
-        riemann_col(b, face, a, bb, 1, total, tp);
-        if (b.turb) {
-          // the whole-face turbulent copy/fix of the reference ends as set by
-          // the last face cell in its loop order
-          double last = riemann_col(b, face, na - 1, nb - 1, 0, total, tp);
-          if (last > 0.) turb_copycol(b, CP_FLAT, face, a, bb);
-          else turb_fixcol(b, p, face, a, bb);
-        }
-      }
-      for (int l = 0; l < b.nv; ++l) {
-        double v0 = q[l * nc + fcell(b, face, 0, a, bb)];
-        q[l * nc + fcell(b, face, -1, a, bb)] = v0;
-        q[l * nc + fcell(b, face, -2, a, bb)] = v0;
-      }
-      break;
-    }
-    case -9: {  // single-block periodic: whole plane, three layers
-      // the reference's array assignment reads its source layers whole
-      // before writing; with one or two cells in the direction they overlap
-      // the destination layers.  Layers g = 0..2 sit at d0 + g*st (ghosts)
-      // and s0 + g*st (their sources) along the face normal's stride st.
-      long d0, s0, st;
-      switch (face) {
-        case 0: d0 = ci(b, -2, a, bb); s0 = ci(b, b.imx - 3, a, bb); st = 1; break;
-        case 1: d0 = ci(b, b.imx, a, bb); s0 = ci(b, 1, a, bb); st = 1; break;
-        case 2: d0 = ci(b, a, -2, bb); s0 = ci(b, a, b.jmx - 3, bb); st = b.pi; break;
-        case 3: d0 = ci(b, a, b.jmx, bb); s0 = ci(b, a, 1, bb); st = b.pi; break;
-        case 4: d0 = ci(b, a, bb, -2); s0 = ci(b, a, bb, b.kmx - 3); st = (long)b.pi * b.pj; break;
-        default: d0 = ci(b, a, bb, b.kmx); s0 = ci(b, a, bb, 1); st = (long)b.pi * b.pj; break;
-      }
-      for (int l = 0; l < b.nv; ++l) {
-        double *v = q + l * nc;
-        const double v0 = v[s0], v1 = v[s0 + st], v2 = v[s0 + 2 * st];
-        v[d0] = v0;
-        v[d0 + st] = v1;
-        v[d0 + 2 * st] = v2;
-      }
-      break;
-    }
     default:
-      break;  // interfaces (>=0) and -10 are filled by the interface exchange
+      return;
   }
+  long cin[4], cgh[3];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) cin[m] = fcell(b, face, m + 1, a, bb);
+#pragma unroll
+  for (int g = 0; g < 3; ++g) cgh[g] = fcell(b, face, -g, a, bb);
+  double in[BC_NV][4], gh[BC_NV][3];
+#pragma unroll
+  for (int l = 0; l < BC_NV; ++l)
+    if (l < b.nv) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) in[l][m] = q[l * nc + cin[m]];
+    }
+#pragma unroll
+  for (int l = 0; l < BC_NV; ++l) {
+    if (l >= b.nv) continue;
+    const int k = r.kind[l];
+    const double a1 = k == BK_SYMM ? b.c1 : 1., a2 = k == BK_SYMM ? b.c2 : k == BK_ANTI ? -1. : 1.,
+                 a3 = k == BK_SYMM ? b.c3 : 0.;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      // ghost layer g takes interior layer g+1 (anti, symm) or layer 1 (flat)
+      const double v1 = k == BK_FLAT ? in[l][0] : in[l][g], v2 = k == BK_FLAT ? in[l][1] : in[l][g + 1];
+      const double w = a2 * v1 - a3 * v2;
+      gh[l][g] = k == BK_FIX ? r.val[l] : a1 == 1. ? w : w / a1;
+    }
+  }
+  unsigned done = 0;  // variables whose ghosts a special rule has filled
+  if (id == -5) {
+    // src/boundary/bc_primitive.f90:1778-1945
+    const double Tw = p.fix[FX_TWALL], R = b.R, gm = b.gm;
+    if (Tw < 0.0) {
+      const double stag = (in[4][0] / (R * in[0][0])) * (1 + (0.5 * (gm - 1.) * gm * in[4][0] / in[0][0]));
+#pragma unroll
+      for (int g = 0; g < 3; ++g) gh[0][g] = gh[4][g] / (R * stag);
+    } else if (Tw > 1.0) {
+#pragma unroll
+      for (int g = 0; g < 3; ++g) gh[0][g] = gh[4][g] / (R * (2 * Tw - (in[4][g] / (R * in[0][g]))));
+    }
+    if (two_eq(b) && !b.kkl) {
+      // src/boundary/bc_primitive.f90:564-643 (Sutherland mu whatever mu_variation)
+      const double T_face = 0.5 * ((gh[4][0] / gh[0][0]) + (in[4][0] / in[0][0])) / b.R;
+      const double mu = b.mu_ref * pow(T_face / b.T_ref, 1.5) * ((b.T_ref + b.S_ref) / (T_face + b.S_ref));
+      const double rm = 0.5 * (gh[0][0] + in[0][0]);
+      const double d2 = 2 * b.dist[cin[0]];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) gh[6][g] = 120 * mu / (rm * 0.075 * (d2 * d2)) - in[6][g];
+      done |= 1u << 6;
+    }
+  } else if (id == -6) {
+    // src/boundary/FT_bc.f90:36-106; j and k faces reflect with the I-face
+    // normal stored at the same index, as the reference does
+    double nx, ny, nz;
+    bnormal(b, face, a, bb, nx, ny, nz);
+    long f;
+    switch (face) {
+      case 0: f = fi(b, 0, 1, a, bb); break;
+      case 1: f = fi(b, 0, b.imx, a, bb); break;
+      case 2: f = fi(b, 0, a, 1, bb); break;
+      case 3: f = fi(b, 0, a, b.jmx, bb); break;
+      case 4: f = fi(b, 0, a, bb, 1); break;
+      default: f = fi(b, 0, a, bb, b.kmx); break;
+    }
+    const double rx = b.fx[0][f], ry = b.fy[0][f], rz = b.fz[0][f];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      const double dot = in[1][g] * nx + in[2][g] * ny + in[3][g] * nz;
+      gh[1][g] = in[1][g] - (2.0 * dot * rx);
+      gh[2][g] = in[2][g] - (2.0 * dot * ry);
+      gh[3][g] = in[3][g] - (2.0 * dot * rz);
+    }
+    done |= 0xe;
+  } else if (riemann) {
+    double c[5], g0[5], nrm[3];
+#pragma unroll
+    for (int l = 0; l < 5; ++l) c[l] = in[l][0];
+    bnormal(b, face, a, bb, nrm[0], nrm[1], nrm[2]);
+    riemann_state(b, face, c, nrm, true, id == -11, p.fix[FX_TP], g0);
+#pragma unroll
+    for (int l = 0; l < 5; ++l) gh[l][0] = gh[l][1] = gh[l][2] = g0[l];
+    done |= 0x1f;
+  }
+#pragma unroll
+  for (int l = 0; l < BC_NV; ++l)
+    if (l < b.nv && (r.kind[l] != BK_LEFT || (done >> l & 1))) {
+#pragma unroll
+      for (int g = 0; g < 3; ++g) q[l * nc + cgh[g]] = gh[l][g];
+    }
+}
+__device__ __forceinline__ void k_bc_face_b(const Blk &b, const Wg &wg, int current_iter) {
+  k_bc_face_b(b, wg.z, (int)(wg.x * 64 + threadIdx.x) - 2, (int)(wg.y * 4 + threadIdx.y) - 2, current_iter);
 }
 
-// edges and corners, src/boundary/bc_primitive.f90:209-224: phase 0 the
-// four lines along i, phase 1 the four lines along k, phase 2 the corners
-__device__ __forceinline__ void k_bc_edges_b(const Blk &b, const Wg &wg, int phase) {
-  int t = wg.x * blockDim.x + threadIdx.x;
+// Edges and corners, src/boundary/bc_primitive.f90:209-224: the four lines
+// along i, then the four along k, then the eight corners, each from the three
+// cells next to it.  One launch takes all three: a line's end cells that a
+// later one overwrites are left out, and what a later one reads of an earlier
+// one (the k lines' and corners' neighbours on the other lines) is formed
+// again from the cells below, which none of the three writes.
+__host__ __device__ inline long edge_cells(const Blk &b) { return 4L * (b.imx + 5) + 4L * (b.kmx + 5) + 8; }
+__device__ __forceinline__ void k_bc_edges_b(const Blk &b, const Wg &wg) {
+  long t = (long)wg.x * blockDim.x + threadIdx.x;
   const int I = b.imx, J = b.jmx, K = b.kmx;
-#define Q(i, j, k) v[ci(b, i, j, k)]
-  if (phase == 0) {
-    int n = I + 5;
-    if (t >= 4 * n * b.nv) return;
-    int l = t / (4 * n), r = t % (4 * n), s = r / n, i = r % n - 2;
-    double *v = b.qp + (long)l * b.nc;
-    if (s == 0) Q(i, 0, 0) = 0.33 * (Q(i, 1, 1) + Q(i, 0, 1) + Q(i, 1, 0));
-    else if (s == 1) Q(i, 0, K) = 0.33 * (Q(i, 1, K - 1) + Q(i, 0, K - 1) + Q(i, 1, K));
-    else if (s == 2) Q(i, J, 0) = 0.33 * (Q(i, J - 1, 1) + Q(i, J, 1) + Q(i, J - 1, 0));
-    else Q(i, J, K) = 0.33 * (Q(i, J - 1, K - 1) + Q(i, J, K - 1) + Q(i, J - 1, K));
-  } else if (phase == 1) {
-    int n = K + 5;
-    if (t >= 4 * n * b.nv) return;
-    int l = t / (4 * n), r = t % (4 * n), s = r / n, k = r % n - 2;
-    double *v = b.qp + (long)l * b.nc;
-    if (s == 0) Q(I, 0, k) = 0.33 * (Q(I - 1, 1, k) + Q(I - 1, 0, k) + Q(I, 1, k));
-    else if (s == 1) Q(0, 0, k) = 0.33 * (Q(1, 1, k) + Q(1, 0, k) + Q(0, 1, k));
-    else if (s == 2) Q(0, J, k) = 0.33 * (Q(1, J - 1, k) + Q(1, J, k) + Q(0, J - 1, k));
-    else Q(I, J, k) = 0.33 * (Q(I - 1, J - 1, k) + Q(I - 1, J, k) + Q(I, J - 1, k));
-  } else {
-    if (t >= 8 * b.nv) return;
-    int l = t / 8, s = t % 8;
-    double *v = b.qp + (long)l * b.nc;
-    switch (s) {
-      case 0: Q(0, 0, 0) = 0.33 * (Q(1, 0, 0) + Q(0, 1, 0) + Q(0, 0, 1)); break;
-      case 1: Q(I, 0, 0) = 0.33 * (Q(I - 1, 0, 0) + Q(I, 1, 0) + Q(I, 0, 1)); break;
-      case 2: Q(0, J, 0) = 0.33 * (Q(1, J, 0) + Q(0, J - 1, 0) + Q(0, J, 1)); break;
-      case 3: Q(0, 0, K) = 0.33 * (Q(1, 0, K) + Q(0, 1, K) + Q(0, 0, K - 1)); break;
-      case 4: Q(I, J, 0) = 0.33 * (Q(I - 1, J, 0) + Q(I, J - 1, 0) + Q(I, J, 1)); break;
-      case 5: Q(I, 0, K) = 0.33 * (Q(I - 1, 0, K) + Q(I, 1, K) + Q(I, 0, K - 1)); break;
-      case 6: Q(0, J, K) = 0.33 * (Q(1, J, K) + Q(0, J - 1, K) + Q(0, J, K - 1)); break;
-      default: Q(I, J, K) = 0.33 * (Q(I - 1, J, K) + Q(I, J - 1, K) + Q(I, J, K - 1)); break;
-    }
+  const long n = edge_cells(b);
+  if (t >= n * b.nv) return;
+  const int l = (int)(t / n);
+  t -= l * n;
+  double *v = b.qp + (long)l * b.nc;
+  auto Q = [&](int i, int j, int k) -> double & { return v[ci(b, i, j, k)]; };
+  // the line along i at (j, k) of i, the line along k at (i, j) of k: jn, kn, in the interior neighbours
+  auto line_i = [&](int i, int j, int k, int jn, int kn) { return 0.33 * (Q(i, jn, kn) + Q(i, j, kn) + Q(i, jn, k)); };
+  auto line_k = [&](int i, int j, int k, int in, int jn) { return 0.33 * (Q(in, jn, k) + Q(in, j, k) + Q(i, jn, k)); };
+  if (t < 4 * (I + 5)) {
+    const int s = (int)(t / (I + 5)), i = (int)(t % (I + 5)) - 2;
+    if (i == 0 || i == I) return;  // the lines along k have these
+    const int j = s < 2 ? 0 : J, k = s & 1 ? K : 0;
+    Q(i, j, k) = line_i(i, j, k, s < 2 ? 1 : J - 1, s & 1 ? K - 1 : 1);
+    return;
   }
-#undef Q
+  t -= 4 * (I + 5);
+  if (t < 4 * (K + 5)) {
+    const int s = (int)(t / (K + 5)), k = (int)(t % (K + 5)) - 2;
+    if (k == 0 || k == K) return;  // the corners
+    const int i = s == 0 || s == 3 ? I : 0, j = s < 2 ? 0 : J;
+    Q(i, j, k) = line_k(i, j, k, i ? I - 1 : 1, j ? J - 1 : 1);
+    return;
+  }
+  t -= 4 * (K + 5);
+  const int i = t & 1 ? I : 0, j = t & 2 ? J : 0, k = t & 4 ? K : 0;
+  const int in = i ? I - 1 : 1, jn = j ? J - 1 : 1, kn = k ? K - 1 : 1;
+  Q(i, j, k) = 0.33 * (line_i(in, j, k, jn, kn) + Q(i, jn, k) + line_k(i, j, kn, in, jn));
 }
 
 }  // namespace fest

@@ -5,11 +5,13 @@
 
 namespace fest {
 
-__global__ void k_bc_face(Blk b, int face0, int current_iter) {
-  k_bc_face_b(b, FEST_WG_HW, face0, current_iter);
+// faces first .. first + gridDim.z - 1
+__global__ void __launch_bounds__(256) k_bc_face(Blk b, int first, int current_iter) {
+  const Wg wg{(int)blockIdx.x, (int)blockIdx.y, first + (int)blockIdx.z, 0};
+  k_bc_face_b(b, wg, current_iter);
 }
-__global__ void k_bc_edges(Blk b, int phase) {
-  k_bc_edges_b(b, FEST_WG_HW, phase);
+__global__ void __launch_bounds__(256) k_bc_edges(Blk b) {
+  k_bc_edges_b(b, FEST_WG_HW);
 }
 
 }  // namespace fest

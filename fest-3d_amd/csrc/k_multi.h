@@ -22,12 +22,12 @@ __global__ void __launch_bounds__(256) km_step_begin(const Blk *__restrict__ blk
   FEST_WALK(k_step_begin_b(b, wg, store_u))
 }
 __global__ void __launch_bounds__(256) km_bc_face(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
-                                                  int n, int face0, int current_iter) {
-  FEST_WALK(k_bc_face_b(b, wg, face0, current_iter))
+                                                  int n, int current_iter) {
+  FEST_WALK(k_bc_face_b(b, wg, current_iter))
 }
 __global__ void __launch_bounds__(256) km_bc_edges(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
-                                                   int n, int phase) {
-  FEST_WALK(k_bc_edges_b(b, wg, phase))
+                                                   int n) {
+  FEST_WALK(k_bc_edges_b(b, wg))
 }
 template <int NG, bool S2003, bool F32 = false>
 __global__ void __launch_bounds__(256) km_grad(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,

@@ -71,3 +71,23 @@ def test_implicit_sweep_tiles(ni, nj, nk, turb):
         g.get_next_solution(it)
     inner = (slice(None),) + (slice(3, -3),) * 3
     assert relerr(g.download("qp")[inner], o.arr("qp")[inner]) <= TOL
+
+
+@pytest.mark.parametrize("bcs", [(-3, -4, -5, -8, -9, -9), (-8, -2, -8, -6, -5, -8), (-9, -9, -6, -5, -8, -4),
+                                 (-1, -11, -9, -9, -6, -6), (-7, -4, -6, -8, -11, -5)])
+@pytest.mark.parametrize("ni,nj,nk", [(3, 4, 5), (4, 3, 9), (5, 7, 3), (6, 4, 4)])
+def test_ghost_launches(ni, nj, nk, bcs):
+    """Every ghost cell, edge and corner after one residual: faces that share
+    a launch and those that may not, directions of three cells (where a face
+    reads the other's ghosts) and more.  Both inflow-fix classes."""
+    case, nodes, q = C.sst_bump(ni, nj, nk, first=0.02)
+    tp = 1.02 * case.p_inf * (1 + 0.2 * case.MInf ** 2) ** 3.5
+    case = dataclasses.replace(case, bc_id=bcs, fix_tp=(tp,) * 6)
+    print("ghosts", ni, nj, nk, bcs, flush=True)
+    g, o = pair(case, nodes, q, True)
+    for it in (1, 3):
+        assert o.residual(it) == 0
+        g.residual(it)
+        a, b = g.download("qp"), o.arr("qp")
+        for l in range(7):
+            assert relerr(a[l], b[l]) <= TOL, (it, l)
