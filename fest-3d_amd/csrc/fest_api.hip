@@ -104,7 +104,7 @@ struct fest_handle {
 // itself and leaves the group unusable (its links point into the block)
 // the phases of a batched group step (k_multi.h), each one launch over the
 // tiles of every block
-enum { PH_BEGIN = 0, PH_BC0, PH_BC1, PH_BC2, PH_BC3, PH_BC4, PH_BC5, PH_EDGES, PH_F32, PH_GRAD, PH_GRAD_BC,
+enum { PH_BEGIN = 0, PH_BC0, PH_BC1, PH_BC2, PH_BC3, PH_BC4, PH_BC5, PH_EDGES, PH_F32, PH_GRAD,
        PH_FLUX_I, PH_FLUX_J, PH_FLUX_K, PH_DT, PH_UPDATE, PH_COUNT };
 
 struct fest_group {
@@ -379,7 +379,6 @@ int launch_grads(fest_handle *h) {
     dim3 gb(cdiv(mx, 64), cdiv(mx, 4), 6);
     {
       KgScope ts(h, KG_GRAD_BC);
-      hipLaunchKernelGGL(k_grad_bc, gb, dim3(64, 4, 1), 0, st, b);
       bool tp = false;
       for (int f = 0; f < 6; ++f) tp |= b.bc[f] == -11;
       // k-kL's mu_t needs no gradients: the ghosts keep the value from the
@@ -1405,11 +1404,6 @@ bool phase_grid(const Blk &b, int ph, dim3 &g, int ti = TILE_I) {
     case PH_EDGES: g = dim3(cdiv(edge_cells(b) * b.nv, 256), 1, 1); return true;
     case PH_F32: g = dim3(cdiv(b.nc * b.nv, 256), 1, 1); return b.fp32 != 0;
     case PH_GRAD: g = dim3(cdiv((long)(b.imx + 1) * (b.jmx + 1), FLAT_BLOCK), b.kmx + 1, 1); return b.mu_ref != 0.0;
-    case PH_GRAD_BC: {
-      const int mx = std::max(std::max(b.imx, b.jmx), b.kmx);
-      g = dim3(cdiv(mx, 64), cdiv(mx, 4), 6);
-      return b.mu_ref != 0.0;
-    }
     case PH_FLUX_I: g = dim3(cdiv(flux_i_span(b), FLUX_I_SPAN), b.kmx - 1, 1); return true;
     case PH_FLUX_J: g = dim3(cdiv(b.imx - 1, ti) * cdiv(b.jmx, tj), b.kmx - 1, 1); return true;
     case PH_FLUX_K: g = dim3(cdiv(b.imx - 1, ti) * cdiv(b.jmx - 1, tj), b.kmx, 1); return true;
@@ -1463,19 +1457,6 @@ int build_lists(fest_group *g, int order) {
         continue;
       }
       if (!phase_grid(b, ph, gr, g->tile_i)) continue;
-      if (ph == PH_GRAD_BC) {
-        // the ghost-gradient rule per face, exact tiles of the face
-        // interior, none on interface faces (k_grad_bc_b leaves those):
-        // the per-block launch's square grid over the largest extent
-        // is mostly idle tiles on uneven blocks
-        for (int z = 0; z < 6; ++z) {
-          if (b.bc[z] >= 0) continue;
-          const unsigned nx = cdiv(face_na(b, z) - 1, 64), ny = cdiv(face_nb(b, z) - 1, 4);
-          for (unsigned y = 0; y < ny; ++y)
-            for (unsigned x = 0; x < nx; ++x) per[n].push_back(WorkItem{(int)n, (int)x, (int)y, z});
-        }
-        continue;
-      }
       for (unsigned z = 0; z < gr.z; ++z)
         for (unsigned y = 0; y < gr.y; ++y)
           for (unsigned x = 0; x < gr.x; ++x) per[n].push_back(WorkItem{(int)n, (int)x, (int)y, (int)z});
@@ -1553,7 +1534,6 @@ int run_group_op_batched(fest_group *g, const StepOp &op, int current_iter) {
         } else {
           KM(PH_GRAD, (km_grad<4, false>), dim3(256));
         }
-        KM(PH_GRAD_BC, km_grad_bc, dim3(64, 4, 1));
       }
       for (int d = 0; d < 3; ++d) {
         const int ph = PH_FLUX_I + d;

@@ -240,11 +240,91 @@ __device__ __forceinline__ void lctm_source(double rho, double tk, double tw, do
   S_gm = (P_gm - D_gm) * vol;
 }
 
+// the face (0..5) whose ghost cell next to its interior (i, j, k) is, or -1
+__device__ __forceinline__ int ghost_face(const Blk &b, int i, int j, int k) {
+  const int gi = i == 0 ? 0 : i == b.imx ? 1 : -1, gj = j == 0 ? 2 : j == b.jmx ? 3 : -1,
+            gk = k == 0 ? 4 : k == b.kmx ? 5 : -1;
+  if ((gi >= 0) + (gj >= 0) + (gk >= 0) != 1) return -1;
+  return gi >= 0 ? gi : gj >= 0 ? gj : gk;
+}
+__device__ __forceinline__ int face_id(const Blk &b, int face) {
+  int id = b.bc[0];
+#pragma unroll
+  for (int f = 1; f < 6; ++f)
+    if (face == f) id = b.bc[f];
+  return id;
+}
+// whether a face's ghost cells take mu_t and F1 from the interior
+// (src/viscosity.f90:407-465; k-kL: -4..-1, -6, -8, -9 and -5, :485-531)
+__device__ __forceinline__ bool visc_rule(const Blk &b, int id) {
+  return (id == -5 || (id <= -1 && id >= -9)) && !(b.kkl && id == -7);
+}
+
+// The ghost cells' gradients, mu_t and F1 on the faces that interior cell
+// (i, j, k) is next to, for boundary ids < 0 (src/gradients.f90:486-676).  Its
+// own gradients gg, mu_t and F1 are all the rules need, so its thread writes
+// them: with a pass of its own over the six faces a stage's gradients took
+// 400 + 83 us at 256x128x128 (SST) and 29 + 22 us at 97x61x45, so 463 and 45.  The reference passes Jfaces/Kfaces to a
+// dummy declared with the I-face extents, so the J/K metrics are read at the
+// I-face linear offset (src/gradients.f90:523-588 calling :591); that is
+// reproduced.
+template <int NG>
+__device__ __forceinline__ void ghost_gradients(const Blk &b, int i, int j, int k, double vol,
+                                                const double (&gg)[NG][3], double mut, double F1) {
+  const long cI = ci(b, i, j, k);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int n = d == 0 ? i : d == 1 ? j : k, N = d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx;
+    if (n != 1 && n != N - 1) continue;
+#pragma unroll 1
+    for (int hi = 0; hi < 2; ++hi) {
+      const int id = hi ? b.bc[2 * d + 1] : b.bc[2 * d];
+      if (n != (hi ? N - 1 : 1) || id >= 0) continue;
+      const double Tw = hi ? b.fix[FX_TWALL][2 * d + 1] : b.fix[FX_TWALL][2 * d];
+      const int fp = hi ? N : 1, g = hi ? N : 0;  // the face and its first ghost layer
+      const long fo = d == 0 ? fi(b, 0, fp, j, k) : d == 1 ? fi(b, 0, i, fp, k) : fi(b, 0, i, j, fp);
+      const long cG = d == 0 ? ci(b, g, j, k) : d == 1 ? ci(b, i, g, k) : ci(b, i, j, g);
+      const long gG = d == 0 ? gri(b, g, j, k) : d == 1 ? gri(b, i, g, k) : gri(b, i, j, g);
+      const double nx = b.fx[d][fo], ny = b.fy[d][fo], nz = b.fz[d][fo], A = b.fA[d][fo];
+      const double c_x = A * nx / vol, c_y = A * ny / vol, c_z = A * nz / vol;
+      const double sig = hi ? -1.0 : 1.0;
+#pragma unroll
+      for (int l = 0; l < NG; ++l) {
+        const double *v = grad_var(b, l);
+        const double dq = v[cI] - v[cG];
+        double ox = sig * dq * c_x, oy = sig * dq * c_y, oz = sig * dq * c_z;
+        const double ix = gg[l][0], iy = gg[l][1], iz = gg[l][2];
+        if (l == 3 && id == -5 && (Tw < 1. && Tw >= 0.)) {
+          ox = -ix; oy = -iy; oz = -iz;
+        }
+        const double dot = (ix * nx) + (iy * ny) + (iz * nz);
+        const double rx = ox + (ix - dot * nx), ry = oy + (iy - dot * ny), rz = oz + (iz - dot * nz);
+        const long o = (long)l * b.ngr + gG;
+        if (!b.g32only) {
+          b.g[0][o] = rx;
+          b.g[1][o] = ry;
+          b.g[2][o] = rz;
+        }
+        if (b.fp32) {
+          b.g32[0][o] = (float)rx;
+          b.g32[1][o] = (float)ry;
+          b.g32[2][o] = (float)rz;
+        }
+      }
+      if (NG >= 5 && visc_rule(b, id)) {
+        b.mut[cG] = id == -5 ? -mut : mut;
+        if (NG >= 6) b.f1[cG] = F1;
+      }
+    }
+  }
+}
+
 // One thread per cell 0..imx x 0..jmx x 0..kmx: all Green-Gauss gradients,
 // then (same cell, gradients in registers) the molecular viscosity, the SST
 // mu_t and F1 (src/viscosity.f90:52-388) and, for interior cells, the SST
-// source.  Interior gradients are final here: the ghost-gradient rule only
-// writes ghost cells.  NG is the number of gradient slots (4 laminar, 6
+// source.  The first ghost cells of a boundary face get the ghost rules' values
+// from the interior cell next to them (ghost_gradients); their own threads
+// keep off what those write.  NG is the number of gradient slots (4 laminar, 6
 // SST); a compile-time count keeps all 3*NG gradients in registers.
 // F32: the FP32 mode when only FP32 gradients are kept (g32only) -- the
 // Green-Gauss sums run in FP32 over the FP32 state copy (Temp from its FP64
@@ -274,6 +354,10 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   const double ivol2 = 1.0 / (2 * vol);
   const long si = 1, sj = b.pi, sk = (long)b.pi * b.pj;
   long gidx = gri(b, i, j, k);
+  const int gface = ghost_face(b, i, j, k), gid = face_id(b, gface);
+  const bool keep_g = gface < 0 || gid >= 0;                 // the gradients are this thread's
+  const bool keep_m = gface < 0 || !visc_rule(b, gid);       // mu_t and F1 are
+  const bool interior = i >= 1 && i <= b.imx - 1 && j >= 1 && j <= b.jmx - 1 && k >= 1 && k <= b.kmx - 1;
   bool bad = false;
   int ndir = (b.kmx > 2) ? 3 : 2;
   double gg[NG][3];
@@ -314,7 +398,7 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
         }
         bad |= isnan(g);
         gg[l][d] = (double)g;
-        b.g32[d][(long)l * b.ngr + gidx] = g;
+        if (keep_g) b.g32[d][(long)l * b.ngr + gidx] = g;
       }
     }
   } else {
@@ -340,8 +424,8 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
       }
       bad |= isnan(g);
       gg[l][d] = g;
-      if (!b.g32only) b.g[d][(long)l * b.ngr + gidx] = g;
-      if (b.fp32) b.g32[d][(long)l * b.ngr + gidx] = (float)g;
+      if (!b.g32only && keep_g) b.g[d][(long)l * b.ngr + gidx] = g;
+      if (b.fp32 && keep_g) b.g32[d][(long)l * b.ngr + gidx] = (float)g;
     }
   }
   }
@@ -363,8 +447,12 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
     const double tk = b.qp[5 * b.nc + c], tkl = b.qp[6 * b.nc + c];
     double mut = pow(0.09, 0.25) * rho * tkl / (fmx(sqrt(tk), 1.e-20));
     if (tkl < 1.e-14 || tk < 1.e-14) mut = 0.0;
-    b.mut[c] = mut;
+    if (keep_m) b.mut[c] = mut;
+    if (interior) ghost_gradients<NG>(b, i, j, k, vol, gg, mut, 0.0);
     return;
+  }
+  if constexpr (NG == 4) {
+    if (interior) ghost_gradients<NG>(b, i, j, k, vol, gg, 0.0, 0.0);
   }
   if constexpr (NG == 6 || NG == 7) {
   double tk = b.qp[5 * b.nc + c], tw = b.qp[6 * b.nc + c];
@@ -374,9 +462,12 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
     const long cl = ci(b, b.imx, b.jmx, b.kmx);
     F1 = lctm_f1(F1, b.qp[cl], b.qp[5 * b.nc + cl], b.dist[c], mu);
   }
-  b.mut[c] = mut;
-  b.f1[c] = F1;
-  if (i >= 1 && i <= b.imx - 1 && j >= 1 && j <= b.jmx - 1 && k >= 1 && k <= b.kmx - 1) {
+  if (keep_m) {
+    b.mut[c] = mut;
+    b.f1[c] = F1;
+  }
+  if (interior) {
+    ghost_gradients<NG>(b, i, j, k, vol, gg, mut, F1);
     double S_k, S_w;
     if constexpr (NG == 7) {
       double S_gm;
@@ -396,8 +487,10 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   }
   if constexpr (NG == 5) {
   double tv = b.qp[5 * b.nc + c];
-  b.mut[c] = sa_mut(rho, tv, mu);
-  if (i >= 1 && i <= b.imx - 1 && j >= 1 && j <= b.jmx - 1 && k >= 1 && k <= b.kmx - 1) {
+  const double mut = sa_mut(rho, tv, mu);
+  if (keep_m) b.mut[c] = mut;
+  if (interior) {
+    ghost_gradients<NG>(b, i, j, k, vol, gg, mut, 0.0);
     // the density gradient over the face sums rho_neighbour + rho
     const double *q0 = b.qp;
     double rf[6] = {q0[c - si] + rho, q0[c - sj] + rho, q0[c - sk] + rho,
@@ -429,81 +522,6 @@ __global__ void __launch_bounds__(256) k_grad(Blk b) {
   k_grad_b<NG, S2003, BC, KKL, F32>(b, FEST_WG_HW);
 }
 
-// mu_t / F1 ghost rules (src/viscosity.f90:407-465), face interiors
-__device__ __forceinline__ void visc_ghost(const Blk &b, int face, int a, int bb) {
-  int id = b.bc[face];
-  if (!(id == -5 || (id <= -1 && id >= -9))) return;
-  if (b.kkl && id == -7) return;  // k-kL: -4..-1, -6, -8, -9 and -5 (src/viscosity.f90:485-531)
-  long cg = fcell(b, face, 0, a, bb), cn = fcell(b, face, 1, a, bb);
-  b.mut[cg] = (id == -5) ? -b.mut[cn] : b.mut[cn];
-  if (b.ng >= 6) b.f1[cg] = b.f1[cn];
-}
-
-
-// ghost-cell gradients on the face interiors of every face with a
-// boundary id < 0.  The reference passes Jfaces/Kfaces to a dummy declared
-// with the I-face extents, so the J/K metrics are read at the I-face linear
-// offset (src/gradients.f90:523-588 calling :591); that is reproduced.
-__device__ __forceinline__ void k_grad_bc_b(const Blk &b, const Wg &wg) {
-  int face = wg.z;
-  int a = wg.x * blockDim.x + threadIdx.x + 1;
-  int bb = wg.y * blockDim.y + threadIdx.y + 1;
-  int na = face_na(b, face), nb = face_nb(b, face);
-  if (a > na - 1 || bb > nb - 1) return;
-  int id = b.bc[face];
-  if (id >= 0) return;
-  if (b.turb) visc_ghost(b, face, a, bb);
-  int d = face >> 1, hi = face & 1;
-  double Tw = b.fix[FX_TWALL][face];
-  // face position and the interior (I) / ghost (G) cells
-  int fi_, fj_, fk_;
-  int N = d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx;
-  int fp = hi ? N : 1;
-  if (d == 0) { fi_ = fp; fj_ = a; fk_ = bb; } else if (d == 1) { fi_ = a; fj_ = fp; fk_ = bb; } else { fi_ = a; fj_ = bb; fk_ = fp; }
-  int Ii = fi_, Ij = fj_, Ik = fk_, Gi = fi_, Gj = fj_, Gk = fk_;
-  if (hi) { if (d == 0) Ii--; else if (d == 1) Ij--; else Ik--; }
-  else { if (d == 0) Gi--; else if (d == 1) Gj--; else Gk--; }
-  long fo = fi(b, 0, fi_, fj_, fk_);  // I-face offset for every direction
-  double nx = b.fx[d][fo], ny = b.fy[d][fo], nz = b.fz[d][fo], A = b.fA[d][fo];
-  long cI = ci(b, Ii, Ij, Ik), cG = ci(b, Gi, Gj, Gk);
-  double vI = b.vol[cI];
-  double c_x = A * nx / vI, c_y = A * ny / vI, c_z = A * nz / vI;
-  double sig = hi ? -1.0 : 1.0;
-  long gI = gri(b, Ii, Ij, Ik), gG = gri(b, Gi, Gj, Gk);
-  double *gx = b.g[0], *gy = b.g[1], *gz = b.g[2];
-  float *hx = b.g32[0], *hy = b.g32[1], *hz = b.g32[2];
-  // the interior gradient: FP64, or its FP32 copy when that is all there is
-  auto gin = [&](int c, long o) -> double {
-    if (b.g32only) return (double)(c == 0 ? hx : c == 1 ? hy : hz)[o];
-    return (c == 0 ? gx : c == 1 ? gy : gz)[o];
-  };
-  for (int l = 0; l < b.ng; ++l) {
-    double dq = b.qp[(long)(l + 1) * b.nc + cI] - b.qp[(long)(l + 1) * b.nc + cG];
-    if (l == 3) dq = b.temp[cI] - b.temp[cG];
-    double ox = sig * dq * c_x, oy = sig * dq * c_y, oz = sig * dq * c_z;
-    long o = (long)l * b.ngr;
-    double ix = gin(0, o + gI), iy = gin(1, o + gI), iz = gin(2, o + gI);
-    if (l == 3 && id == -5 && (Tw < 1. && Tw >= 0.)) {
-      ox = -ix; oy = -iy; oz = -iz;
-    }
-    double dot = (ix * nx) + (iy * ny) + (iz * nz);
-    const double rx = ox + (ix - dot * nx), ry = oy + (iy - dot * ny), rz = oz + (iz - dot * nz);
-    if (!b.g32only) {
-      gx[o + gG] = rx;
-      gy[o + gG] = ry;
-      gz[o + gG] = rz;
-    }
-    if (b.fp32) {
-      hx[o + gG] = (float)rx;
-      hy[o + gG] = (float)ry;
-      hz[o + gG] = (float)rz;
-    }
-  }
-}
-__global__ void k_grad_bc(Blk b) {
-  k_grad_bc_b(b, FEST_WG_HW);
-}
-
 // FP32 copy of the padded state for the FP32 face sweeps
 __device__ __forceinline__ void k_to_f32_b(const Blk &b, const Wg &wg) {
   long t = (long)wg.x * blockDim.x + threadIdx.x;
@@ -523,8 +541,8 @@ __global__ void k_g32_widen(Blk b) {
 
 // A -11 face has no mu_t / F1 ghost rule (src/viscosity.f90:284-339,
 // 409-465 list -1..-9): its ghost cells keep the SST values
-// calculate_viscosity computes there, from the ghost gradients k_grad_bc has
-// written.  Launched after k_grad_bc, only when an SST block has a -11 face.
+// calculate_viscosity computes there, from the ghost gradients k_grad has
+// written.  Launched after it, only when an SST block has a -11 face.
 __device__ __forceinline__ void k_mut_ghost_tp_b(const Blk &b, const Wg &wg) {
   int face = wg.z;
   int a = wg.x * blockDim.x + threadIdx.x + 1;

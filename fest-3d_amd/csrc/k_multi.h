@@ -34,10 +34,6 @@ __global__ void __launch_bounds__(256) km_grad(const Blk *__restrict__ blks, con
                                                int n) {
   FEST_WALK((k_grad_b<NG, S2003, false, false, F32>(b, wg)))
 }
-__global__ void __launch_bounds__(256) km_grad_bc(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
-                                                  int n) {
-  FEST_WALK(k_grad_bc_b(b, wg))
-}
 __global__ void __launch_bounds__(256) km_dt(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
                                              int n) {
   FEST_WALK(k_dt_b(b, wg))

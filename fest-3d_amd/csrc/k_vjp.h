@@ -577,7 +577,7 @@ __global__ void __launch_bounds__(256) k_vjp_nodes(Blk b, const double *__restri
 // viscosities, and the average of their gradients of u, v, w, T.  T is
 // p/(R rho) of the state; the gradients are the Green-Gauss sums of
 // k_grad_b (of u, v, w and the temperature plane) and, in the ghost cells
-// of boundary faces, the rule of k_grad_bc_b; the viscosities come from
+// of boundary faces, the rule of ghost_gradients; the viscosities come from
 // Sutherland's law of T when the case uses it (src/viscosity.f90), else they
 // are constants.  The temperature plane is the state's p/(R rho) at upload
 // (src/update.f90:170, taken before the ghost refill): its interior cells
@@ -740,7 +740,7 @@ __global__ void __launch_bounds__(256) k_vjp_visc_gather(Blk b, const double *__
   for (int e = 0; e < 12; ++e) gb[(long)e * b.ngr + g] = 0.5 * acc[5 + e];
 }
 
-// the transpose of k_grad_bc_b on one face (boundary ids < 0), one thread
+// the transpose of ghost_gradients on one face (boundary ids < 0), one thread
 // per face-interior column: the ghost cell's gradient adjoint goes to the
 // interior cell's gradient and to the differences of the two cells' values
 // it reads, then is cleared (the Green-Gauss sum the rule overwrites is
