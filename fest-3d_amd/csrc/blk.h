@@ -144,19 +144,37 @@ __device__ __forceinline__ bool flat_ij(int ni, int nj, int &i, int &j, int blk)
   return j < nj;
 }
 
-// Tiled variant: each 256-thread block is a TI (i) x 256/TI (j) tile --
-// 64 x 4 by default, 32 x 8 for narrow blocks of a batched group -- tiles
-// numbered i-fastest in blockIdx.x, blockIdx.y = k.  Sweeps whose stencil
-// runs along j or k keep whole rows of one i-range in one block.
-constexpr int TILE_I = 64, TILE_J = 4;
-template <int TI = TILE_I>
-__device__ __forceinline__ bool tile_ij(int ni, int nj, int &i, int &j, int blk) {
-  constexpr int TJ = 256 / TI;
-  const int ntx = (ni + TI - 1) / TI;
+// Tiled variant: each 256-thread block is a ti (i) x 256/ti (j) tile, ti a
+// power of two from 16 to 64, tiles numbered i-fastest in blockIdx.x,
+// blockIdx.y = k.  Sweeps whose stencil runs along j or k keep whole rows of
+// one i-range in one block.
+constexpr int TILE_I = 64;
+__device__ __forceinline__ bool tile_ij(int ni, int nj, int &i, int &j, int blk, int ti) {
+  const int ntx = (ni + ti - 1) / ti, lg = __builtin_ctz(ti);
   const int tx = blk % ntx, ty = blk / ntx;
-  i = tx * TI + ((int)threadIdx.x & (TI - 1));
-  j = ty * TJ + ((int)threadIdx.x / TI);
+  i = tx * ti + ((int)threadIdx.x & (ti - 1));
+  j = ty * (256 >> lg) + ((int)threadIdx.x >> lg);
   return i < ni && j < nj;
+}
+// The tile width, at most `most`, that covers rows of ni cells, nj of them,
+// with the least work: the padded area, an eighth more for 32-wide tiles'
+// 16-wide ones, whose waves hold four rows (more of them next to a boundary,
+// shorter runs of memory).  97x61 cells take 64 (the sweeps 98 us at
+// 97x61x45 SST, 113 in 16-wide tiles), the 16..48-cell blocks of the chain 16
+// or 32 (211 -> 163 us).
+inline int tile_width(int ni, int nj, int most) {
+  int best = most;
+  double cost = 0;
+  for (int ti = most; ti >= 16; ti /= 2) {
+    const int tj = 256 / ti;
+    const double c = (double)((ni + ti - 1) / ti * ti) * ((nj + tj - 1) / tj * tj) *
+                     (ti == 64 ? 1.0 : ti == 32 ? 1.03 : 1.16);
+    if (ti == most || c < cost) {
+      best = ti;
+      cost = c;
+    }
+  }
+  return best;
 }
 
 // stride of the padded cell arrays along direction d

@@ -105,7 +105,7 @@ struct fest_handle {
 // the phases of a batched group step (k_multi.h), each one launch over the
 // tiles of every block
 enum { PH_BEGIN = 0, PH_BC0, PH_BC1, PH_BC2, PH_BC3, PH_BC4, PH_BC5, PH_EDGES, PH_F32, PH_GRAD,
-       PH_FLUX_I, PH_FLUX_J, PH_FLUX_K, PH_DT, PH_UPDATE, PH_COUNT };
+       PH_FLUX, PH_DT, PH_UPDATE, PH_COUNT };
 
 struct fest_group {
   std::vector<fest_handle *> blocks;
@@ -127,7 +127,7 @@ struct fest_group {
   int grid_cap = 0;       // work-groups per batched launch; 0: one per tile
   int order = 0;          // 0: tiles block by block; 1: the blocks' tiles interleaved
   int lists_order = -1;   // order the device lists were built in
-  int tile_i = TILE_I;    // i width of the j/k sweeps' face tiles: 64 (x 4) or 32 (x 8)
+  int tile_i = TILE_I;    // widest j/k face tile: 64 (x 4) or 32 (x 8)
   int lists_tile = -1;    // tile width the device lists were built with
   Blk *d_blks = nullptr;
   double *d_norms = nullptr;  // NORM_SLOTS doubles per block: norms, then the block's share
@@ -275,12 +275,6 @@ int check_err(fest_handle *h) {
   return fail(h, FEST_E_CONFIG, "device error bits 0x%x", e);
 }
 
-// grid of 64 x 4 tiles over an (ni x nj x nk) box (the kernels use tile_ij)
-inline void tiles(long ni, long nj, long nk, dim3 &g, dim3 &t, int pad8) {
-  t = dim3(TILE_I * TILE_J, 1, 1);
-  g = dim3(plane_slots((long)cdiv(ni, TILE_I) * cdiv(nj, TILE_J), pad8), (unsigned)nk, 1);
-}
-
 // The launches of a block's faces, in the reference's order imin, imax, jmin,
 // ...: the first and the last face of each.  Faces share a launch when none
 // reads what another writes.  A direction's two faces read its interior
@@ -395,6 +389,23 @@ int launch_grads(fest_handle *h) {
   return 0;
 }
 
+// the launch of a block's face sweeps: blocks of FLUX_I_SPAN consecutive
+// padded-plane offsets for the i sweep, face tiles for the others
+Sweeps sweep_slots(const Blk &b, int pad8, int widest = TILE_I) {
+  Sweeps s;
+  const int ti = s.ti = tile_width(b.imx - 1, b.jmx - 1, widest), tj = 256 / ti;
+  s.S[0] = (int)plane_slots(cdiv(flux_i_span(b), FLUX_I_SPAN), pad8);
+  s.S[1] = (int)plane_slots((long)cdiv(b.imx - 1, ti) * cdiv(b.jmx, tj), pad8);
+  s.S[2] = (int)plane_slots((long)cdiv(b.imx - 1, ti) * cdiv(b.jmx - 1, tj), pad8);
+  return s;
+}
+void launch_block_sweeps(const Blk &b, const Sweeps &s, int only, int count, hipStream_t st, int store_csnd) {
+  if (b.nv == 8) launch_sweeps<8>(b, s, only, count, st, store_csnd);
+  else if (b.nv == 7) launch_sweeps<7>(b, s, only, count, st, store_csnd);
+  else if (b.nv == 6) launch_sweeps<6>(b, s, only, count, st, store_csnd);
+  else launch_sweeps<5>(b, s, only, count, st, store_csnd);
+}
+
 // C2..C9(+C10 in k_update): ghosts, gradients/viscosity, face fluxes
 int launch_residual_front(fest_handle *h, int current_iter, int store_csnd) {
   Blk &b = h->b;
@@ -406,23 +417,14 @@ int launch_residual_front(fest_handle *h, int current_iter, int store_csnd) {
   }
   LAUNCHCHK(h);
   if (int rc = launch_grads(h)) return rc;
-  dim3 g, t;
-  // the i sweep: blocks of FLUX_I_SPAN consecutive padded-plane offsets
-  g = dim3(plane_slots(cdiv(flux_i_span(b), FLUX_I_SPAN), b.xcd_remap), (unsigned)(b.kmx - 1), 1);
-  t = dim3(FLUX_I_SPAN, 1, 1);
-  {
-    KgScope ts(h, KG_FLUX_I);
-    launch_flux<0>(b, g, t, st, store_csnd);
-  }
-  tiles(b.imx - 1, b.jmx, b.kmx - 1, g, t, b.xcd_remap);
-  {
-    KgScope ts(h, KG_FLUX_J);
-    launch_flux<1>(b, g, t, st, store_csnd);
-  }
-  tiles(b.imx - 1, b.jmx - 1, b.kmx, g, t, b.xcd_remap);
-  {
-    KgScope ts(h, KG_FLUX_K);
-    launch_flux<2>(b, g, t, st, store_csnd);
+  const Sweeps s = sweep_slots(b, b.xcd_remap);
+  if (h->timed & (1u << KG_FLUX_I | 1u << KG_FLUX_J | 1u << KG_FLUX_K)) {
+    for (int d = 0; d < 3; ++d) {
+      KgScope ts(h, KG_FLUX_I + d);
+      launch_block_sweeps(b, s, d, s.S[d] * (b.kmx - 1 + (d == 2)), st, store_csnd);
+    }
+  } else {
+    launch_block_sweeps(b, s, -1, (s.S[0] + s.S[1] + s.S[2]) * (b.kmx - 1) + s.S[2], st, store_csnd);
   }
   LAUNCHCHK(h);
   return 0;
@@ -1397,16 +1399,12 @@ int group_exchange(fest_group *g) {
 
 // the per-block launch grid of a phase (as launch_residual_front and the
 // step operations lay it out); false when the block has no tiles in it
-bool phase_grid(const Blk &b, int ph, dim3 &g, int ti = TILE_I) {
-  const int tj = 256 / ti;
+bool phase_grid(const Blk &b, int ph, dim3 &g) {
   switch (ph) {
     case PH_BEGIN: g = dim3(cdiv(b.nc, 256), 1, 1); return true;
     case PH_EDGES: g = dim3(cdiv(edge_cells(b) * b.nv, 256), 1, 1); return true;
     case PH_F32: g = dim3(cdiv(b.nc * b.nv, 256), 1, 1); return b.fp32 != 0;
     case PH_GRAD: g = dim3(cdiv((long)(b.imx + 1) * (b.jmx + 1), FLAT_BLOCK), b.kmx + 1, 1); return b.mu_ref != 0.0;
-    case PH_FLUX_I: g = dim3(cdiv(flux_i_span(b), FLUX_I_SPAN), b.kmx - 1, 1); return true;
-    case PH_FLUX_J: g = dim3(cdiv(b.imx - 1, ti) * cdiv(b.jmx, tj), b.kmx - 1, 1); return true;
-    case PH_FLUX_K: g = dim3(cdiv(b.imx - 1, ti) * cdiv(b.jmx - 1, tj), b.kmx, 1); return true;
     case PH_DT: case PH_UPDATE:
       g = dim3(cdiv((long)(b.imx - 1) * (b.jmx - 1), FLAT_BLOCK), b.kmx - 1, 1);
       return true;
@@ -1456,13 +1454,34 @@ int build_lists(fest_group *g, int order) {
         }
         continue;
       }
-      if (!phase_grid(b, ph, gr, g->tile_i)) continue;
+      if (ph == PH_FLUX) {
+        const Sweeps s = sweep_slots(b, 0, g->tile_i);
+        for (int y = 0; y < b.kmx; ++y)
+          for (int d = y < b.kmx - 1 ? 0 : 2; d < 3; ++d)
+            for (int x = 0; x < s.S[d]; ++x) per[n].push_back(WorkItem{(int)n, x, y, d | s.ti << 8});
+        continue;
+      }
+      if (!phase_grid(b, ph, gr)) continue;
       for (unsigned z = 0; z < gr.z; ++z)
         for (unsigned y = 0; y < gr.y; ++y)
           for (unsigned x = 0; x < gr.x; ++x) per[n].push_back(WorkItem{(int)n, (int)x, (int)y, (int)z});
     }
     g->ph_off[ph] = (int)all.size();
-    if (order == 0) {
+    if (order == 0 && (ph == PH_GRAD || ph == PH_FLUX || ph == PH_UPDATE)) {
+      // Work-groups go to the 8 XCDs in turn, so the list is dealt in eights:
+      // each XCD gets a slab of k planes of every block, plane after plane,
+      // and finds the neighbouring rows, planes and directions in its own L2
+      std::vector<WorkItem> slab[8];
+      for (size_t n = 0; n < per.size(); ++n) {
+        const int planes = per[n].empty() ? 1 : per[n].back().y + 1;
+        for (const WorkItem &it : per[n]) slab[it.y * 8 / planes].push_back(it);
+      }
+      size_t mx = 0;
+      for (auto &v : slab) mx = std::max(mx, v.size());
+      for (size_t t = 0; t < mx; ++t)
+        for (auto &v : slab)
+          if (t < v.size()) all.push_back(v[t]);
+    } else if (order == 0) {
       for (auto &v : per) all.insert(all.end(), v.begin(), v.end());
     } else {
       // round robin over the blocks, one tile of each in turn
@@ -1535,13 +1554,11 @@ int run_group_op_batched(fest_group *g, const StepOp &op, int current_iter) {
           KM(PH_GRAD, (km_grad<4, false>), dim3(256));
         }
       }
-      for (int d = 0; d < 3; ++d) {
-        const int ph = PH_FLUX_I + d;
-        if (!g->ph_n[ph]) continue;
-        const WorkItem *items = g->d_items + g->ph_off[ph];
-        if (d == 0) launch_flux_batched<0>(b0, st, g->d_blks, items, g->ph_n[ph], grid(ph), g->tile_i, op.flags);
-        else if (d == 1) launch_flux_batched<1>(b0, st, g->d_blks, items, g->ph_n[ph], grid(ph), g->tile_i, op.flags);
-        else launch_flux_batched<2>(b0, st, g->d_blks, items, g->ph_n[ph], grid(ph), g->tile_i, op.flags);
+      if (g->ph_n[PH_FLUX]) {
+        const WorkItem *items = g->d_items + g->ph_off[PH_FLUX];
+        const int n = g->ph_n[PH_FLUX];
+        if (b0.nv == 7) launch_sweeps_batched<7>(b0, st, g->d_blks, items, n, grid(PH_FLUX), op.flags);
+        else launch_sweeps_batched<5>(b0, st, g->d_blks, items, n, grid(PH_FLUX), op.flags);
       }
       break;
     case OP_DT: KM(PH_DT, km_dt, dim3(256)); break;

@@ -1,7 +1,7 @@
-// flux_launch.h -- launchers of the face-sweep kernels (k_flux, km_flux),
-// compiled in their own translation unit (flux_launch.hip): the sweeps'
-// many specialisations (direction x variables x reconstruction x
-// precision x tile) then build beside the rest of the library.
+// flux_launch.h -- launchers of the face-sweep kernels (k_sweeps, km_sweeps),
+// compiled in translation units of their own, one per variable count
+// (flux_launch.hip): the sweeps' many specialisations (variables x
+// reconstruction x precision) then build beside the rest of the library.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -11,27 +11,16 @@ namespace fest {
 
 struct WorkItem;
 
-// sweep D of one block: k_flux<D, NV, RECON, FLAT, T> for the block's
-// variable count, reconstruction and precision (FLAT on the k faces of a
-// 2-D grid), grid g of blocks t, on stream st
-template <int D>
-void launch_flux(const Blk &b, dim3 g, dim3 t, hipStream_t st, int store_csnd);
+// the face sweeps of one block of NV variables (k_sweeps), count work-groups:
+// all three (only -1) or one
+template <int NV>
+void launch_sweeps(const Blk &b, const struct Sweeps &s, int only, int count, hipStream_t st, int store_csnd);
 
-// sweep D over the work list of a batched group step (n items, `grid`
-// work-groups; the j and k sweeps in tile_i x 256/tile_i face tiles); b0 is
-// any block of the group (they share one kernel variant)
-template <int D>
-void launch_flux_batched(const Blk &b0, hipStream_t st, const Blk *blks, const WorkItem *items, int n,
-                         unsigned grid, int tile_i, int store_csnd);
-
-extern template void launch_flux<0>(const Blk &, dim3, dim3, hipStream_t, int);
-extern template void launch_flux<1>(const Blk &, dim3, dim3, hipStream_t, int);
-extern template void launch_flux<2>(const Blk &, dim3, dim3, hipStream_t, int);
-extern template void launch_flux_batched<0>(const Blk &, hipStream_t, const Blk *, const WorkItem *, int, unsigned,
-                                            int, int);
-extern template void launch_flux_batched<1>(const Blk &, hipStream_t, const Blk *, const WorkItem *, int, unsigned,
-                                            int, int);
-extern template void launch_flux_batched<2>(const Blk &, hipStream_t, const Blk *, const WorkItem *, int, unsigned,
-                                            int, int);
+// the face sweeps over the work list of a batched group step of blocks of NV
+// (5 or 7) variables (n items, `grid` work-groups); b0 is any block of the
+// group (they share one kernel variant)
+template <int NV>
+void launch_sweeps_batched(const Blk &b0, hipStream_t st, const Blk *blks, const WorkItem *items, int n,
+                           unsigned grid, int store_csnd);
 
 }  // namespace fest

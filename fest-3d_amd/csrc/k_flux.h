@@ -619,8 +619,8 @@ __host__ __device__ inline long flux_i_span(const Blk &b) {
   return (b.imx + 2) + (long)(b.jmx + 1) * b.pi - flux_i_first(b) + 1;
 }
 
-template <int D, int NV, int RECON, bool FLAT, typename T, int TI = TILE_I>
-__device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int store_csnd) {
+template <int D, int NV, int RECON, bool FLAT, typename T>
+__device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int store_csnd) {
   using M = FaceMath<T>;
   const int ii = D == 0, jj = D == 1, kk = D == 2;
   int i, j;
@@ -655,8 +655,7 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int store_c
     if (!active) return;
     lds_row = &sq[0][t + 3];
   } else {
-    // j, k sweeps: 64 x 4 tiles
-    if (!tile_ij<TI>(b.imx - 1 + ii, b.jmx - 1 + jj, i, j, blk)) return;
+    if (!tile_ij(b.imx - 1, b.jmx - 1 + jj, i, j, blk, ti)) return;
     i += 1;
     j += 1;
     if (k > b.kmx - 1 + kk) return;
@@ -729,9 +728,46 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int store_c
   if (bad) atomicOr(b.err, ERR_NAN_FLUX);
   if (store_csnd) b.csnd[D][o] = (double)csf;
 }
-template <int D, int NV, int RECON, bool FLAT = false, typename T = double>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_flux(Blk b, int store_csnd) {
-  k_flux_b<D, NV, RECON, FLAT, T>(b, FEST_WG_HW, store_csnd);
+
+// The three sweeps of one launch, k plane after k plane: a plane's work-groups
+// are S[0] of the i sweep, S[1] of the j sweep and S[2] of the k sweep (the
+// last k faces follow by themselves).  The sweeps share the state, gradients,
+// viscosities and cell centres, 248 of their 338 bytes a face (SST); plane by
+// plane an XCD finds most of it in its L2 again, having just worked on the
+// same rows in another direction.  Three launches read it from memory three
+// times, and take 10 us each however small the block.
+struct Sweeps {
+  int S[3];  // slots per plane of each sweep (a multiple of 8 under the XCD-aware order)
+  int ti;    // width of the j and k sweeps' tiles (tile_width)
+};
+template <int NV, int RECON, bool FLAT, typename T>
+__device__ __forceinline__ void k_sweeps_b(const Blk &b, int dir, const Wg &wg, int ti, int store_csnd) {
+  if (dir == 0) k_flux_b<0, NV, RECON, false, T>(b, wg, ti, store_csnd);
+  else if (dir == 1) k_flux_b<1, NV, RECON, false, T>(b, wg, ti, store_csnd);
+  else k_flux_b<2, NV, RECON, FLAT, T>(b, wg, ti, store_csnd);
+}
+// only: all three sweeps (-1) or one of them (timed runs)
+template <int NV, int RECON, bool FLAT, typename T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_sweeps(Blk b, Sweeps s, int only, int store_csnd) {
+  const int w = (int)blockIdx.x, P = s.S[0] + s.S[1] + s.S[2], last = P * (b.kmx - 1);
+  int dir = only, plane, x;
+  if (only >= 0) {
+    const int S = only == 0 ? s.S[0] : only == 1 ? s.S[1] : s.S[2];
+    plane = w / S;
+    x = w % S;
+  } else if (w >= last) {
+    dir = 2;
+    plane = b.kmx - 1;
+    x = w - last;
+  } else {
+    plane = w / P;
+    x = w % P;
+    dir = x < s.S[0] ? 0 : x < s.S[0] + s.S[1] ? 1 : 2;
+    x -= dir == 0 ? 0 : dir == 1 ? s.S[0] : s.S[0] + s.S[1];
+  }
+  const int S = dir == 0 ? s.S[0] : dir == 1 ? s.S[1] : s.S[2];
+  k_sweeps_b<NV, RECON, FLAT, T>(b, dir, Wg{x, plane, 0, S}, s.ti, store_csnd);
 }
 
 }  // namespace fest

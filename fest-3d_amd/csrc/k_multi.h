@@ -6,7 +6,7 @@
 // takes tiles t, t + gridDim.x, ... in turn (a persistent launch).  The
 // tile bodies are the per-block kernels' own (k_*_b), so a tile computes
 // exactly what the per-block launch computes for it.  The face sweeps'
-// batched kernel, km_flux, is in k_flux_walk.h.
+// batched kernel, km_sweeps, is in k_flux_walk.h.
 #pragma once
 #include "blk.h"
 #include "k_bc.h"

@@ -337,11 +337,12 @@ int fest_group_get_next_solution(fest_group *g, int current_iter, double cfl);
  *               time steps; RK4, RK2 or none), else FEST_E_CONFIG.
  *   "grid_cap"  work-groups per batched launch, each walking the work list
  *               (a persistent launch); 0 (default): one per tile.
- *   "order"     0: each block's tiles together; 1: the blocks' tiles
- *               interleaved.
- *   "tile_i"    64 (default) or 32: the j and k face sweeps of a batched
- *               step in 64 x 4 or 32 x 8 face tiles (narrow blocks leave
- *               fewer lanes idle in the narrower tile).
+ *   "order"     0: each block's tiles together (those of the gradients, the
+ *               sweeps and the update by slabs of k planes, one per XCD); 1:
+ *               the blocks' tiles interleaved.
+ *   "tile_i"    64 (default) or 32: the widest face tile of the j and k
+ *               sweeps of a batched step, 64 x 4 or 32 x 8 (each block takes
+ *               the tile up to that width that leaves the fewest lanes idle).
  * The results do not depend on the schedule. */
 int fest_group_set_option(fest_group *g, const char *name, long value);
 /* Autotuner of the group step's schedule (no counterpart in the reference):
