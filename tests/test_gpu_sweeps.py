@@ -91,3 +91,34 @@ def test_ghost_launches(ni, nj, nk, bcs):
         a, b = g.download("qp"), o.arr("qp")
         for l in range(7):
             assert relerr(a[l], b[l]) <= TOL, (it, l)
+
+
+@pytest.mark.parametrize("turb", ["none", "kkl"])
+@pytest.mark.parametrize("ni,nj,nk", [(3, 3, 3), (5, 4, 7), (64, 4, 3), (33, 65, 3), (127, 63, 35)])
+def test_norm_sums(ni, nj, nk, turb):
+    """The residual norms from one cell a thread and a mostly empty wave to
+    more cells than 1024 work-groups have threads (127 x 63 x 35), against
+    extended-precision sums of the downloaded residue and face fluxes.  Any
+    order of m additions of positive terms is within m 2^-53 of the exact sum
+    (3e-11 here); the imbalance is held to that of its terms' magnitudes."""
+    if turb == "none":
+        case, nodes, q = C.laminar_box(ni, nj, nk)
+    else:
+        case, nodes, q = C.sst_bump(ni, nj, nk, turb=turb, recon="muscl", first=0.02)
+    g = GpuBlock(case)
+    g.set_grid(nodes, wall_dist=turb != "none")
+    g.upload_state(q)
+    g.residual(1)
+    out = g.download("residue", "F", "G", "H")
+    norms = g.resnorm()
+    m = ni * nj * nk
+    v, rho, p = case.vel_mag, case.rho_inf, case.p_inf
+    scale = [rho * v] + 3 * [rho * v * v] + [0.5 * rho * v**3 + case.gm / (case.gm - 1) * p]
+    for l, s in enumerate(scale):
+        r = out["residue"][l].astype(np.longdouble)
+        assert norms[1 + l] == pytest.approx(float(np.sqrt((r * r).sum())) / s, rel=m * 2.0**-53 + 1e-14, abs=0)
+    F, G, H = (out[n][0].astype(np.longdouble) for n in "FGH")
+    ends = [F[:, :, 0], -F[:, :, -1], G[:, 0, :], -G[:, -1, :], H[0], -H[-1]]
+    exact = abs(float(sum(e.sum() for e in ends)))
+    mag = float(sum(abs(e).sum() for e in ends))
+    assert abs(norms[0] - exact) <= (m * 2.0**-53 + 1e-14) * mag
