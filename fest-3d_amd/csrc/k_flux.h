@@ -115,6 +115,39 @@ struct FaceMath {
                         T(-1.0) * Up1 + T(5.0) * U0 + T(2.0) * Um1, T(2.0) * U0 + T(5.0) * Um1 - T(1.0) * Um2);
   }
 
+  // The FP64 WENO5 of the two cells of a face in differences of neighbours,
+  // d1..d5 of the six cells w0..w5.  A candidate polynomial less the cell's
+  // value, a smoothness indicator's terms and the second differences are sums
+  // of one to three of them, the second differences' squares serve both cells,
+  // and the quotient is a correction to the cell's value, which needs no last
+  // remainder step: 85 FP64 instructions for a variable's two states, 122 as
+  // two calls of the forms above.
+  // weno_diff: the correction of a cell, times its 6, from the indicators (with
+  // eps) and the differences in the order towards the face.
+  static __device__ __forceinline__ double weno_diff(double B1, double B2, double B3, double d1, double d2, double d3,
+                                                     double d4) {
+    const double D1 = B1 * B1, D2 = B2 * B2, D3 = B3 * B3;
+    // the weights 1, 6, 3 over D1, D2, D3, times D1 D2 D3; e2 is half of its
+    const double t = 3.0 * D1, e1 = D2 * D3, e2 = t * D3, e3 = t * D2;
+    const double num = e1 * (5.0 * d2 - 2.0 * d1) + e2 * (2.0 * d2 + 4.0 * d3) + e3 * (4.0 * d3 - d4);
+    const double den = (e1 + 2.0 * e2) + e3;
+    double y = __builtin_amdgcn_rcp(den);
+    y = __builtin_fma(__builtin_fma(-den, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-den, y, 1.0), y, y);
+    return num * y;
+  }
+  static __device__ __forceinline__ void weno_pair(double w0, double w1, double w2, double w3, double w4, double w5,
+                                                   double &L, double &R) {
+    const double eps = 1e-6, c = 13.0 / 12.0, sixth = 1.0 / 6.0;
+    const double d1 = w1 - w0, d2 = w2 - w1, d3 = w3 - w2, d4 = w4 - w3, d5 = w5 - w4;
+    const double s1 = d2 - d1, s2 = d3 - d2, s3 = d4 - d3, s4 = d5 - d4;
+    const double S1 = eps + c * (s1 * s1), S2 = eps + c * (s2 * s2), S3 = eps + c * (s3 * s3), S4 = eps + c * (s4 * s4);
+    const double hL = d2 + d3, hR = d3 + d4;
+    const double l1 = 0.5 * s1 + d2, l3 = d3 - 0.5 * s3, r1 = d4 - 0.5 * s4, r3 = d3 + 0.5 * s2;
+    L = w2 + sixth * weno_diff(S1 + l1 * l1, S2 + (0.25 * hL) * hL, S3 + l3 * l3, d1, d2, d3, d4);
+    R = w3 - sixth * weno_diff(S4 + r1 * r1, S3 + (0.25 * hR) * hR, S2 + r3 * r3, d5, d4, d3, d2);
+  }
+
   // WENO for non-uniform grids (weno_NM.f90:59-121): a21, a10, a01, a12
   // are the volume blends V(m)/(V(m-1)+V(m)) of the cell's stencil, m = -1..2
   // relative to the cell.  Polynomials and indicators as the reference, the
@@ -271,48 +304,52 @@ struct FaceMath {
     const bool bmin = minbc < 0 && minbc != -10, bmax = maxbc < 0 && maxbc != -10;
     return (bmin && n <= (b.ppm_flag ? 2 : 1)) || (bmax && n >= (b.ppm_flag ? N - 1 : N));
   }
-  // face_states of a face away from the boundary rules, without a branch:
-  // the stencil loads of one variable can be in flight while another's
-  // arithmetic runs, and the two cells' common differences are formed once
+  // the cells of a face's stencil that a reconstruction reads
   template <int RECON, typename Q>
-  static __device__ __forceinline__ void inner_states(const Blk &b, int d, int l, const Q *u, long s, const Aux &ax,
+  static __device__ __forceinline__ void stencil(const Q *u, long s, T (&w)[6]) {
+    constexpr int m0 = RECON == 0 ? 2 : RECON == 1 ? 1 : 0;
+#pragma unroll
+    for (int m = m0; m < 6 - m0; ++m) w[m] = T(u[(long)(m - 3) * s]);
+  }
+  // face_states of a face away from the boundary rules, from its stencil,
+  // without a branch; the two cells' common differences are formed once
+  template <int RECON>
+  static __device__ __forceinline__ void inner_states(const Blk &b, int d, int l, const T (&w)[6], const Aux &ax,
                                                       T &L, T &R) {
-    auto w = [u, s](int m) { return T(u[(long)(m - 3) * s]); };
     const int sw = (l >= 5) ? b.tlim[d] : b.lim[d];
     T dummy;
     if constexpr (RECON == 0) {
-      L = w(2);
-      R = w(3);
+      L = w[2];
+      R = w[3];
     } else if constexpr (RECON == 1) {
-      const T w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4);
-      muscl_cell(w1, w2, w3, sw, L, dummy, b.valb);
-      muscl_cell(w2, w3, w4, sw, dummy, R, b.valb);
+      muscl_cell(w[1], w[2], w[3], sw, L, dummy, b.valb);
+      muscl_cell(w[2], w[3], w[4], sw, dummy, R, b.valb);
       if (ax.pb) {
-        L = w2 + (ax.pdL * (L - w2));
-        R = w3 - (ax.pdR * (w3 - R));
+        L = w[2] + (ax.pdL * (L - w[2]));
+        R = w[3] - (ax.pdR * (w[3] - R));
       }
     } else if constexpr (RECON == 2) {
-      const T w0 = w(0), w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4), w5 = w(5);
-      const T f0 = ppm_face(w0, w1, w2, w3), f1 = ppm_face(w1, w2, w3, w4), f2 = ppm_face(w2, w3, w4, w5);
+      const T f0 = ppm_face(w[0], w[1], w[2], w[3]), f1 = ppm_face(w[1], w[2], w[3], w[4]), f2 = ppm_face(w[2], w[3], w[4], w[5]);
       T lo = f0, up = f1;
-      if (b.lim[d] == 1) ppm_extrema(w2, up, lo);
+      if (b.lim[d] == 1) ppm_extrema(w[2], up, lo);
       L = up;
       lo = f1;
       up = f2;
-      if (b.lim[d] == 1) ppm_extrema(w3, up, lo);
+      if (b.lim[d] == 1) ppm_extrema(w[3], up, lo);
       R = lo;
       if (ax.pb) {
-        L = w2 + (ax.pdL * (L - w2));
-        R = w3 - (ax.pdR * (w3 - R));
+        L = w[2] + (ax.pdL * (L - w[2]));
+        R = w[3] - (ax.pdR * (w[3] - R));
       }
     } else {
-      const T w0 = w(0), w1 = w(1), w2 = w(2), w3 = w(3), w4 = w(4), w5 = w(5);
-      if constexpr (RECON == 3) {
-        L = weno_up(w0, w1, w2, w3, w4);
-        R = weno_lo(w1, w2, w3, w4, w5);
+      if constexpr (RECON == 3 && std::is_same<T, double>::value) {
+        weno_pair(w[0], w[1], w[2], w[3], w[4], w[5], L, R);
+      } else if constexpr (RECON == 3) {
+        L = weno_up(w[0], w[1], w[2], w[3], w[4]);
+        R = weno_lo(w[1], w[2], w[3], w[4], w[5]);
       } else {
-        L = weno_nm(w0, w1, w2, w3, w4, ax.A[0], ax.A[1], ax.A[2], ax.A[3], true);
-        R = weno_nm(w1, w2, w3, w4, w5, ax.A[1], ax.A[2], ax.A[3], ax.A[4], false);
+        L = weno_nm(w[0], w[1], w[2], w[3], w[4], ax.A[0], ax.A[1], ax.A[2], ax.A[3], true);
+        R = weno_nm(w[1], w[2], w[3], w[4], w[5], ax.A[1], ax.A[2], ax.A[3], ax.A[4], false);
       }
     }
   }
@@ -467,45 +504,99 @@ struct FaceMath {
   // k faces of a 2-D grid, where the reference skips the SST viscous flux
   // (src/viscous.f90:101-105).  NV 6 is Spalart-Allmaras: its nu-tilde flux
   // runs on every face (src/viscous.f90:94-97, 570-656)
+  // FP32 mode reads the FP32 copy of the gradients
+  using GS = typename std::conditional<sizeof(T) == sizeof(float), const float, const double>::type;
+  // one variable's gradient on both sides of a face, as loaded
+  struct Grad {
+    typename std::remove_const<GS>::type a[3][2];
+  };
+  static __device__ __forceinline__ void grad_load(const Blk &b, int l, long gL, long gR, Grad &g) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const GS *p;
+      if constexpr (sizeof(T) == sizeof(float)) p = b.g32[d] + l * b.ngr;
+      else p = b.g[d] + l * b.ngr;
+      g.a[d][0] = p[gL];
+      g.a[d][1] = p[gR];
+    }
+  }
+  // the face gradient: the two sides' average, its component along the line
+  // of the centres replaced by del / |line|
+  static __device__ __forceinline__ void face_grad(const Grad &g, T del, T delx, T dely, T delz, T id2, T (&r)[3]) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) r[d] = T(0.5) * (T(g.a[d][0]) + T(g.a[d][1]));
+    T ncmp = (del - (r[0] * delx + r[1] * dely + r[2] * delz)) * id2;
+    r[0] = r[0] + ncmp * delx;
+    r[1] = r[1] + ncmp * dely;
+    r[2] = r[2] + ncmp * delz;
+  }
+  // what is loaded before the fence is asked for before what follows it is
+  // computed.  The order is written out because the compiler, short of
+  // registers, asks for each variable's inputs when their use has come (PPM
+  // and WENO sweeps: 10 waits of a whole memory latency a face), or not, on a
+  // change of two instructions.  With stencils one variable ahead and the
+  // viscous flux's inputs one gradient ahead, all three sweeps of 256 x 128 x
+  // 128 (SST, WENO5) take 1205 -> 1090 us, of 384 x 192 x 128 (PPM) 2630 ->
+  // 2380 us; two or three variables ahead 1130 us, the gradients asked for
+  // before the inviscid flux 1175 us and up, with spills.  4.3 GB pass at 4.0
+  // TB/s then.  FP32, whose registers suffice, is left to the compiler.
+  static __device__ __forceinline__ void fence() {
+    if constexpr (std::is_same<T, double>::value) __builtin_amdgcn_sched_barrier(0);
+  }
   template <int NV>
   static __device__ __forceinline__ void visc_face(const Blk &b, long c, long cm, long gL, long gR, T nx, T ny, T nz,
                                                    T A, bool laminar_only, T (&v)[NV]) {
     const double *qp = b.qp;
     const long nc = b.nc;
-    const T delx = T(b.cx[c] - b.cx[cm]), dely = T(b.cy[c] - b.cy[cm]), delz = T(b.cz[c] - b.cz[cm]);
+    const double x0 = b.cx[cm], x1 = b.cx[c], y0 = b.cy[cm], y1 = b.cy[c], z0 = b.cz[cm], z1 = b.cz[c];
+    double q0[5], q1[5];
+#pragma unroll
+    for (int l = 0; l < 5; ++l) {
+      q0[l] = qp[l * nc + cm];
+      q1[l] = qp[l * nc + c];
+    }
+    Grad gu, gv, gw, gt;
+    grad_load(b, 0, gL, gR, gu);
+    fence();
+    const T delx = T(x1 - x0), dely = T(y1 - y0), delz = T(z1 - z0);
     T d2 = delx * delx + dely * dely + delz * delz;
     T id2 = tdiv(T(1.0), d2);  // normal_comp*del/d_LR = (del_phi - grad.del)*del/d_LR^2
-    // FP32 mode reads the FP32 copy of the gradients
-    using GS = typename std::conditional<sizeof(T) == sizeof(float), const float, const double>::type;
-    GS *gx, *gy, *gz;
-    if constexpr (sizeof(T) == sizeof(float)) {
-      gx = b.g32[0]; gy = b.g32[1]; gz = b.g32[2];
-    } else {
-      gx = b.g[0]; gy = b.g[1]; gz = b.g[2];
-    }
-    const long ngr = b.ngr;
+    const double T_LE = q0[4] / (q0[0] * b.R);
+    const double T_RE = q1[4] / (q1[0] * b.R);
+    T del[4] = {T(q1[1] - q0[1]), T(q1[2] - q0[2]), T(q1[3] - q0[3]), T(T_RE - T_LE)};
+    T uf = T(0.5) * (T(q0[1]) + T(q1[1]));
+    T vf = T(0.5) * (T(q0[2]) + T(q1[2]));
+    T wf = T(0.5) * (T(q0[3]) + T(q1[3]));
+    grad_load(b, 1, gL, gR, gv);
+    grad_load(b, 2, gL, gR, gw);
+    fence();
     T gr[4][3];
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      gr[l][0] = T(0.5) * (T(gx[l * ngr + gL]) + T(gx[l * ngr + gR]));
-      gr[l][1] = T(0.5) * (T(gy[l * ngr + gL]) + T(gy[l * ngr + gR]));
-      gr[l][2] = T(0.5) * (T(gz[l * ngr + gL]) + T(gz[l * ngr + gR]));
+    face_grad(gu, del[0], delx, dely, delz, id2, gr[0]);
+    const double mu0 = b.mu[cm], mu1 = b.mu[c];
+    double mt0 = 0.0, mt1 = 0.0;
+    if (NV >= 6) {
+      mt0 = b.mut[cm];
+      mt1 = b.mut[c];
     }
-    const double T_LE = qp[4 * nc + cm] / (qp[cm] * b.R);
-    const double T_RE = qp[4 * nc + c] / (qp[c] * b.R);
-    T del[4] = {T(qp[nc + c] - qp[nc + cm]), T(qp[2 * nc + c] - qp[2 * nc + cm]), T(qp[3 * nc + c] - qp[3 * nc + cm]),
-                T(T_RE - T_LE)};
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      T ncmp = (del[l] - (gr[l][0] * delx + gr[l][1] * dely + gr[l][2] * delz)) * id2;
-      gr[l][0] = gr[l][0] + ncmp * delx;
-      gr[l][1] = gr[l][1] + ncmp * dely;
-      gr[l][2] = gr[l][2] + ncmp * delz;
+    grad_load(b, 3, gL, gR, gt);
+    fence();
+    face_grad(gv, del[1], delx, dely, delz, id2, gr[1]);
+    face_grad(gw, del[2], delx, dely, delz, id2, gr[2]);
+    // the turbulence variables' inputs
+    Grad g5, g6;
+    double k0 = 0.0, k1 = 0.0, w0 = 0.0, w1 = 0.0, f0 = 0.0, f1 = 0.0;
+    const bool two_eq = NV >= 7 && (!laminar_only || b.kkl);
+    if (NV == 6 || two_eq) {
+      grad_load(b, 4, gL, gR, g5);
+      k0 = qp[5 * nc + cm];
+      k1 = qp[5 * nc + c];
     }
-    T mu_f = T(0.5) * (T(b.mu[cm]) + T(b.mu[c]));
+    fence();
+    face_grad(gt, del[3], delx, dely, delz, id2, gr[3]);
+    T mu_f = T(0.5) * (T(mu0) + T(mu1));
     // compute_viscous_fluxes_laminar takes mu_t whenever the run is turbulent
     // (src/viscous.f90:270-277)
-    T mut_f = (NV >= 6) ? T(0.5) * (T(b.mut[cm]) + T(b.mut[c])) : T(0.0);
+    T mut_f = (NV >= 6) ? T(0.5) * (T(mt0) + T(mt1)) : T(0.0);
     T tm = mu_f + mut_f;
     T dudx = gr[0][0], dudy = gr[0][1], dudz = gr[0][2];
     T dvdx = gr[1][0], dvdy = gr[1][1], dvdz = gr[1][2];
@@ -519,9 +610,14 @@ struct FaceMath {
     T Tyz = tm * (dwdy + dvdz);
     T K_heat = (mu_f * T(b.iPr) + mut_f * T(b.itPr)) * T(b.cpR);
     T Qx = K_heat * gr[3][0], Qy = K_heat * gr[3][1], Qz = K_heat * gr[3][2];
-    T uf = T(0.5) * (T(qp[nc + cm]) + T(qp[nc + c]));
-    T vf = T(0.5) * (T(qp[2 * nc + cm]) + T(qp[2 * nc + c]));
-    T wf = T(0.5) * (T(qp[3 * nc + cm]) + T(qp[3 * nc + c]));
+    if (two_eq) {
+      grad_load(b, 5, gL, gR, g6);
+      w0 = qp[6 * nc + cm];
+      w1 = qp[6 * nc + c];
+      f0 = b.f1[cm];
+      f1 = b.f1[c];
+    }
+    fence();
     v[0] = T(0.0);
     v[1] = (Txx * nx + Txy * ny + Txz * nz) * A;
     v[2] = (Txy * nx + Tyy * ny + Tyz * nz) * A;
@@ -536,63 +632,43 @@ struct FaceMath {
     if constexpr (NV == 6) {
       // nu-tilde diffusion with (mu + rho_f nu~_f) / sigma, sigma = 2/3; the
       // quotient taken as a product with 1.5 (within an ulp of it)
-      T g0 = T(0.5) * (T(gx[4 * ngr + gL]) + T(gx[4 * ngr + gR]));
-      T g1 = T(0.5) * (T(gy[4 * ngr + gL]) + T(gy[4 * ngr + gR]));
-      T g2 = T(0.5) * (T(gz[4 * ngr + gL]) + T(gz[4 * ngr + gR]));
-      T ncmp = (T(qp[5 * nc + c] - qp[5 * nc + cm]) - (g0 * delx + g1 * dely + g2 * delz)) * id2;
-      g0 = g0 + ncmp * delx;
-      g1 = g1 + ncmp * dely;
-      g2 = g2 + ncmp * delz;
-      T rhof = T(0.5) * (T(qp[cm]) + T(qp[c]));
-      T mtv = T(0.5) * (T(qp[5 * nc + cm]) + T(qp[5 * nc + c])) * rhof;
-      v[NV == 6 ? 5 : 0] = (A * ((mu_f + mtv) * (g0 * nx + g1 * ny + g2 * nz))) * T(1.5);
+      T g[3];
+      face_grad(g5, T(k1 - k0), delx, dely, delz, id2, g);
+      T rhof = T(0.5) * (T(q0[0]) + T(q1[0]));
+      T mtv = T(0.5) * (T(k0) + T(k1)) * rhof;
+      v[NV == 6 ? 5 : 0] = (A * ((mu_f + mtv) * (g[0] * nx + g[1] * ny + g[2] * nz))) * T(1.5);
     }
-    if (NV >= 7 && (!laminar_only || b.kkl)) {
+    if (two_eq) {
       // SST k / omega diffusion and the -2/3 rho k stress, src/viscous.f90:328-447;
       // k-kL's has sigma_k = sigma_phi = 1 and runs on the k faces of a 2-D
       // grid too (:450-567, :106-109)
-      T gt[2][3];
-#pragma unroll
-      for (int l = 0; l < 2; ++l) {
-        gt[l][0] = T(0.5) * (T(gx[(4 + l) * ngr + gL]) + T(gx[(4 + l) * ngr + gR]));
-        gt[l][1] = T(0.5) * (T(gy[(4 + l) * ngr + gL]) + T(gy[(4 + l) * ngr + gR]));
-        gt[l][2] = T(0.5) * (T(gz[(4 + l) * ngr + gL]) + T(gz[(4 + l) * ngr + gR]));
-      }
-      T dt2[2] = {T(qp[5 * nc + c] - qp[5 * nc + cm]), T(qp[6 * nc + c] - qp[6 * nc + cm])};
-#pragma unroll
-      for (int l = 0; l < 2; ++l) {
-        T ncmp = (dt2[l] - (gt[l][0] * delx + gt[l][1] * dely + gt[l][2] * delz)) * id2;
-        gt[l][0] = gt[l][0] + ncmp * delx;
-        gt[l][1] = gt[l][1] + ncmp * dely;
-        gt[l][2] = gt[l][2] + ncmp * delz;
-      }
+      T gk[3], go[3];
+      face_grad(g5, T(k1 - k0), delx, dely, delz, id2, gk);
+      face_grad(g6, T(w1 - w0), delx, dely, delz, id2, go);
       // k-kL leaves F1 at 0 and sets sigma_w2 to 1, so both blends are 1
-      T F1 = T(0.5) * (T(b.f1[cm]) + T(b.f1[c]));
+      T F1 = T(0.5) * (T(f0) + T(f1));
       T sigma_kf = T(0.85) * F1 + T(1.0) * (T(1.0) - F1);
       T sigma_wf = T(0.5) * F1 + T(b.sigma_w2) * (T(1.0) - F1);
-      T rhof = T(0.5) * (T(qp[cm]) + T(qp[c]));
-      T tkf = T(0.5) * (T(qp[5 * nc + cm]) + T(qp[5 * nc + c]));
+      T rhof = T(0.5) * (T(q0[0]) + T(q1[0]));
+      T tkf = T(0.5) * (T(k0) + T(k1));
       T Tkk = -(T(2.0) * rhof * tkf * (T(1.0) / T(3.0)));
       v[1] = v[1] + Tkk * nx * A;
       v[2] = v[2] + Tkk * ny * A;
       v[3] = v[3] + Tkk * nz * A;
-      T kfl = A * ((mu_f + sigma_kf * mut_f) * (gt[0][0] * nx + gt[0][1] * ny + gt[0][2] * nz));
+      T kfl = A * ((mu_f + sigma_kf * mut_f) * (gk[0] * nx + gk[1] * ny + gk[2] * nz));
       v[4] = v[4] + kfl;
       v[NV >= 7 ? 5 : 0] = kfl;
-      v[NV >= 7 ? 6 : 0] = A * ((mu_f + sigma_wf * mut_f) * (gt[1][0] * nx + gt[1][1] * ny + gt[1][2] * nz));
+      v[NV >= 7 ? 6 : 0] = A * ((mu_f + sigma_wf * mut_f) * (go[0] * nx + go[1] * ny + go[2] * nz));
     }
     if constexpr (NV == 8) {
       // lctm2015's intermittency: (mu + mu_t) grad(gamma), no sigma, none on
       // the k faces of a 2-D grid (src/viscous.f90:114-128, 659-746)
       if (!laminar_only) {
-        T g0 = T(0.5) * (T(gx[6 * ngr + gL]) + T(gx[6 * ngr + gR]));
-        T g1 = T(0.5) * (T(gy[6 * ngr + gL]) + T(gy[6 * ngr + gR]));
-        T g2 = T(0.5) * (T(gz[6 * ngr + gL]) + T(gz[6 * ngr + gR]));
-        T ncmp = (T(qp[7 * nc + c] - qp[7 * nc + cm]) - (g0 * delx + g1 * dely + g2 * delz)) * id2;
-        g0 = g0 + ncmp * delx;
-        g1 = g1 + ncmp * dely;
-        g2 = g2 + ncmp * delz;
-        v[NV - 1] = A * ((mu_f + mut_f) * (g0 * nx + g1 * ny + g2 * nz));
+        Grad g7;
+        T g[3];
+        grad_load(b, 6, gL, gR, g7);
+        face_grad(g7, T(qp[7 * nc + c] - qp[7 * nc + cm]), delx, dely, delz, id2, g);
+        v[NV - 1] = A * ((mu_f + mut_f) * (g[0] * nx + g[1] * ny + g[2] * nz));
       }
     }
   }
@@ -619,6 +695,8 @@ __host__ __device__ inline long flux_i_span(const Blk &b) {
   return (b.imx + 2) + (long)(b.jmx + 1) * b.pi - flux_i_first(b) + 1;
 }
 
+// stencils that are on their way while a variable is reconstructed (see fence)
+constexpr int AHEAD = 1;
 template <int D, int NV, int RECON, bool FLAT, typename T>
 __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int store_csnd) {
   using M = FaceMath<T>;
@@ -684,9 +762,10 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int
     }
     if constexpr (RECON == 4) M::nm_blends(b.vol + c, s, ax);
     // FP64 j and k sweeps: the boundary rules apart, the other faces without
-    // a branch.  At 256x128x128 (SST, WENO5) flux_j 482 -> 409 us, flux_k 479
-    // -> 408 us; the i sweep, whose stencils come from LDS, loses by it (439
-    // -> 466 us), and FP32 keeps the one form its results are defined by.
+    // a branch.  At 256x128x128 (SST, WENO5), each alone, flux_j 482 -> 409 us,
+    // flux_k 479 -> 408 us; the i sweep, whose stencils come from LDS, loses by
+    // it (439 -> 466 us; 97 x 61 x 45, all three, 98 -> 103 us), and FP32 keeps
+    // the one form its results are defined by.
     constexpr bool split = D != 0 && std::is_same<T, double>::value;
     if (!split || M::template edge_face<RECON>(b, D, n, N)) {
 #pragma unroll
@@ -696,9 +775,16 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int
         else M::template face_states<RECON>(b, D, n, N, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
       }
     } else {
+      T w[AHEAD + 1][6];
 #pragma unroll
-      for (int l = 0; l < nv; ++l)
-        M::template inner_states<RECON>(b, D, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
+      for (int l = 0; l < AHEAD; ++l) M::template stencil<RECON>(qsrc + (long)l * b.nc + c, s, w[l]);
+#pragma unroll
+      for (int l = 0; l < nv; ++l) {
+        if (l + AHEAD < nv)
+          M::template stencil<RECON>(qsrc + (long)(l + AHEAD) * b.nc + c, s, w[(l + AHEAD) % (AHEAD + 1)]);
+        M::fence();
+        M::template inner_states<RECON>(b, D, l, w[l % (AHEAD + 1)], ax, qL[l], qR[l]);
+      }
     }
     if (store_csnd) csf = T(0.5) * (tsqrt(T(b.gm) * qL[4] / qL[0]) + tsqrt(T(b.gm) * qR[4] / qR[0]));
     const T zero = T((n == 1) ? (double)b.mz[D][0] : (n == N) ? (double)b.mz[D][1] : 1.0);
