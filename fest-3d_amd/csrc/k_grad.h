@@ -11,6 +11,8 @@
 // the unfused reference order by rounding only, far inside the 1e-12 parity
 // bound, and the FP64 instruction count, which bounds these kernels, drops
 #pragma clang fp contract(fast)
+#include <type_traits>
+
 #include "blk.h"
 #include "k_bc.h"
 
@@ -264,8 +266,8 @@ __device__ __forceinline__ bool visc_rule(const Blk &b, int id) {
 // (i, j, k) is next to, for boundary ids < 0 (src/gradients.f90:486-676).  Its
 // own gradients gg, mu_t and F1 are all the rules need, so its thread writes
 // them: with a pass of its own over the six faces a stage's gradients took
-// 400 + 83 us at 256x128x128 (SST) and 29 + 22 us at 97x61x45, so 463 and 45.  The reference passes Jfaces/Kfaces to a
-// dummy declared with the I-face extents, so the J/K metrics are read at the
+// 400 + 83 us at 256x128x128 (SST) and 29 + 22 us at 97x61x45, together 435 and
+// 40.  The reference passes Jfaces/Kfaces to a dummy declared with the I-face extents, so the J/K metrics are read at the
 // I-face linear offset (src/gradients.f90:523-588 calling :591); that is
 // reproduced.
 template <int NG>
@@ -276,25 +278,34 @@ __device__ __forceinline__ void ghost_gradients(const Blk &b, int i, int j, int 
   for (int d = 0; d < 3; ++d) {
     const int n = d == 0 ? i : d == 1 ? j : k, N = d == 0 ? b.imx : d == 1 ? b.jmx : b.kmx;
     if (n != 1 && n != N - 1) continue;
+    // a wave's lanes at either end take one pass together; a direction of one
+    // cell has both faces and takes two
 #pragma unroll 1
-    for (int hi = 0; hi < 2; ++hi) {
+    for (int hi = n != 1; hi < 2; hi += N == 2 ? 1 : 2) {
       const int id = hi ? b.bc[2 * d + 1] : b.bc[2 * d];
-      if (n != (hi ? N - 1 : 1) || id >= 0) continue;
+      if (id >= 0) continue;
       const double Tw = hi ? b.fix[FX_TWALL][2 * d + 1] : b.fix[FX_TWALL][2 * d];
       const int fp = hi ? N : 1, g = hi ? N : 0;  // the face and its first ghost layer
       const long fo = d == 0 ? fi(b, 0, fp, j, k) : d == 1 ? fi(b, 0, i, fp, k) : fi(b, 0, i, j, fp);
       const long cG = d == 0 ? ci(b, g, j, k) : d == 1 ? ci(b, i, g, k) : ci(b, i, j, g);
       const long gG = d == 0 ? gri(b, g, j, k) : d == 1 ? gri(b, i, g, k) : gri(b, i, j, g);
       const double nx = b.fx[d][fo], ny = b.fy[d][fo], nz = b.fz[d][fo], A = b.fA[d][fo];
-      const double c_x = A * nx / vol, c_y = A * ny / vol, c_z = A * nz / vol;
-      const double sig = hi ? -1.0 : 1.0;
+      double vI[NG], vG[NG];
 #pragma unroll
       for (int l = 0; l < NG; ++l) {
-        const double *v = grad_var(b, l);
-        const double dq = v[cI] - v[cG];
+        vI[l] = grad_var(b, l)[cI];
+        vG[l] = grad_var(b, l)[cG];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const double c_x = A * nx / vol, c_y = A * ny / vol, c_z = A * nz / vol;
+      const double sig = hi ? -1.0 : 1.0;
+      const bool wall = id == -5 && (Tw < 1. && Tw >= 0.);
+#pragma unroll
+      for (int l = 0; l < NG; ++l) {
+        const double dq = vI[l] - vG[l];
         double ox = sig * dq * c_x, oy = sig * dq * c_y, oz = sig * dq * c_z;
         const double ix = gg[l][0], iy = gg[l][1], iz = gg[l][2];
-        if (l == 3 && id == -5 && (Tw < 1. && Tw >= 0.)) {
+        if (l == 3 && wall) {
           ox = -ix; oy = -iy; oz = -iz;
         }
         const double dot = (ix * nx) + (iy * ny) + (iz * nz);
@@ -339,8 +350,7 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   long f0 = fi(b, 0, i, j, k), f1 = fi(b, 0, i + 1, j, k);
   long g0 = fi(b, 1, i, j, k), g1 = fi(b, 1, i, j + 1, k);
   long h0 = fi(b, 2, i, j, k), h1 = fi(b, 2, i, j, k + 1);
-  double Ai0 = b.fA[0][f0], Ai1 = b.fA[0][f1], Aj0 = b.fA[1][g0], Aj1 = b.fA[1][g1];
-  double Ak0 = b.fA[2][h0], Ak1 = b.fA[2][h1];
+  double A[6] = {b.fA[0][f0], b.fA[1][g0], b.fA[2][h0], b.fA[0][f1], b.fA[1][g1], b.fA[2][h1]};
   double n[3][6];  // [component][face]
   n[0][0] = b.fx[0][f0]; n[1][0] = b.fy[0][f0]; n[2][0] = b.fz[0][f0];
   n[0][1] = b.fx[1][g0]; n[1][1] = b.fy[1][g0]; n[2][1] = b.fz[1][g0];
@@ -349,91 +359,104 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   n[0][4] = b.fx[1][g1]; n[1][4] = b.fy[1][g1]; n[2][4] = b.fz[1][g1];
   n[0][5] = b.fx[2][h1]; n[1][5] = b.fy[2][h1]; n[2][5] = b.fz[2][h1];
   double vol = b.vol[c];
-  // one reciprocal for all 3*NG quotients by 2V (the reference divides each;
-  // the product differs from the quotient by at most one ulp)
-  const double ivol2 = 1.0 / (2 * vol);
-  const long si = 1, sj = b.pi, sk = (long)b.pi * b.pj;
+  const long st[7] = {0, -1, -(long)b.pi, -(long)b.pi * b.pj, 1, b.pi, (long)b.pi * b.pj};
+  // a variable's cell and its six neighbours, as stored
+  using V = typename std::conditional<F32, float, double>::type;
+  auto load = [&](int l, V (&w)[7]) {
+#pragma unroll
+    for (int m = 0; m < 7; ++m) {
+      if constexpr (F32) w[m] = l == 3 ? (float)b.temp[c + st[m]] : b.q32[(long)(l + 1) * b.nc + c + st[m]];
+      else w[m] = grad_var(b, l)[c + st[m]];
+    }
+  };
+  // Every variable's neighbours are asked for while the one before is summed,
+  // the tail's inputs during the last, and nothing is stored before the last
+  // sum: loads and stores retire in order, so a load behind a store waits for
+  // it too.  With each variable loaded, summed and stored in turn the waits of
+  // a whole memory latency were one a variable: 256
+  // x 128 x 128 (SST) 460 -> 435 us (1.7 GB, 3.9 TB/s), 128 x 96 x 64 (SA) 99
+  // -> 83 us, 97 x 61 x 45 44 -> 40 us, 64 x 64 x 4 (laminar) 10.8 -> 9.0 us.
+  // It takes 142 registers (SST), 3 waves a SIMD; held to 4 it spills (479 us).
+  V w[2][7];
+  load(0, w[0]);
   long gidx = gri(b, i, j, k);
   const int gface = ghost_face(b, i, j, k), gid = face_id(b, gface);
   const bool keep_g = gface < 0 || gid >= 0;                 // the gradients are this thread's
   const bool keep_m = gface < 0 || !visc_rule(b, gid);       // mu_t and F1 are
   const bool interior = i >= 1 && i <= b.imx - 1 && j >= 1 && j <= b.jmx - 1 && k >= 1 && k <= b.kmx - 1;
+  __builtin_amdgcn_sched_barrier(0);
+  // one reciprocal for all 3*NG quotients by 2V (the reference divides each;
+  // the product differs from the quotient by at most one ulp)
+  const double ivol2 = 1.0 / (2 * vol);
   bool bad = false;
   int ndir = (b.kmx > 2) ? 3 : 2;
   double gg[NG][3];
-  if constexpr (F32) {
-    float nf[3][6], Af[6] = {(float)Ai0, (float)Aj0, (float)Ak0, (float)Ai1, (float)Aj1, (float)Ak1};
+  // the weights of the six face sums: signed n A, FP64's over 2V
+  V m[3][6], Af[6];
+  const V iv2 = (V)ivol2;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+  for (int f = 0; f < 6; ++f) {
+    Af[f] = (V)A[f];
+    const double s = f < 3 ? -(A[f] * ivol2) : A[f] * ivol2;
 #pragma unroll
-      for (int f = 0; f < 6; ++f) nf[d][f] = (float)n[d][f];
-    const float iv2 = (float)ivol2;
-#pragma unroll
-    for (int l = 0; l < NG; ++l) {
-      float vc, vmi, vmj, vmk, vpi, vpj, vpk;
-      if (l == 3) {
-        const double *v = b.temp;
-        vc = (float)v[c]; vmi = (float)v[c - si]; vmj = (float)v[c - sj]; vmk = (float)v[c - sk];
-        vpi = (float)v[c + si]; vpj = (float)v[c + sj]; vpk = (float)v[c + sk];
-      } else {
-        const float *v = b.q32 + (long)(l + 1) * b.nc;
-        vc = v[c]; vmi = v[c - si]; vmj = v[c - sj]; vmk = v[c - sk];
-        vpi = v[c + si]; vpj = v[c + sj]; vpk = v[c + sk];
-      }
-      const float sm_i = vmi + vc, sm_j = vmj + vc, sm_k = vmk + vc;
-      const float sp_i = vpi + vc, sp_j = vpj + vc, sp_k = vpk + vc;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        float g;
-        if (d < ndir) {
-          g = -(sm_i * nf[d][0] * Af[0]);
-          g = g - sm_j * nf[d][1] * Af[1];
-          g = g - sm_k * nf[d][2] * Af[2];
-          g = g + sp_i * nf[d][3] * Af[3];
-          g = g + sp_j * nf[d][4] * Af[4];
-          g = g + sp_k * nf[d][5] * Af[5];
-          g = g * iv2;
-        } else {
-          g = 0.0f;
-        }
-        bad |= isnan(g);
-        gg[l][d] = (double)g;
-        if (keep_g) b.g32[d][(long)l * b.ngr + gidx] = g;
-      }
-    }
-  } else {
+    for (int d = 0; d < 3; ++d) m[d][f] = F32 ? (V)n[d][f] : (V)(n[d][f] * s);
+  }
+  double rho, p, dist = 0.0;
 #pragma unroll
   for (int l = 0; l < NG; ++l) {
-    const double *v = grad_var(b, l);
-    double vc = v[c];
-    double sm_i = v[c - si] + vc, sm_j = v[c - sj] + vc, sm_k = v[c - sk] + vc;
-    double sp_i = v[c + si] + vc, sp_j = v[c + sj] + vc, sp_k = v[c + sk] + vc;
+    if (l + 1 < NG) {
+      load(l + 1, w[(l + 1) & 1]);
+    } else {
+      rho = b.qp[c];
+      p = b.qp[4 * b.nc + c];
+      if (NG >= 5) dist = b.dist[c];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const V(&v)[7] = w[l & 1];
+    const V sm_i = v[1] + v[0], sm_j = v[2] + v[0], sm_k = v[3] + v[0];
+    const V sp_i = v[4] + v[0], sp_j = v[5] + v[0], sp_k = v[6] + v[0];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      double g;
-      if (d < ndir) {
-        g = -(sm_i * n[d][0] * Ai0);
-        g = g - sm_j * n[d][1] * Aj0;
-        g = g - sm_k * n[d][2] * Ak0;
-        g = g + sp_i * n[d][3] * Ai1;
-        g = g + sp_j * n[d][4] * Aj1;
-        g = g + sp_k * n[d][5] * Ak1;
-        g = g * ivol2;
+      V g;
+      if constexpr (F32) {
+        g = -(sm_i * m[d][0] * Af[0]);
+        g = g - sm_j * m[d][1] * Af[1];
+        g = g - sm_k * m[d][2] * Af[2];
+        g = g + sp_i * m[d][3] * Af[3];
+        g = g + sp_j * m[d][4] * Af[4];
+        g = g + sp_k * m[d][5] * Af[5];
+        g = g * iv2;
       } else {
-        g = 0.0;
+        g = sm_i * m[d][0];
+        g = g + sm_j * m[d][1];
+        g = g + sm_k * m[d][2];
+        g = g + sp_i * m[d][3];
+        g = g + sp_j * m[d][4];
+        g = g + sp_k * m[d][5];
       }
+      if (d >= ndir) g = V(0);
       bad |= isnan(g);
-      gg[l][d] = g;
-      if (!b.g32only && keep_g) b.g[d][(long)l * b.ngr + gidx] = g;
-      if (b.fp32 && keep_g) b.g32[d][(long)l * b.ngr + gidx] = (float)g;
+      gg[l][d] = (double)g;
     }
   }
+  if (keep_g) {
+    if (!F32 && !b.g32only) {
+#pragma unroll
+      for (int l = 0; l < NG; ++l)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) b.g[d][(long)l * b.ngr + gidx] = gg[l][d];
+    }
+    if (F32 || b.fp32) {
+#pragma unroll
+      for (int l = 0; l < NG; ++l)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) b.g32[d][(long)l * b.ngr + gidx] = (float)gg[l][d];
+    }
   }
   if (bad) atomicOr(b.err, ERR_NAN_GRAD);
-  double rho = b.qp[c];
   double mu;
   if (b.mu_suth) {
-    double T = b.qp[4 * b.nc + c] / (rho * b.R);
+    double T = p / (rho * b.R);
     const double x = T / b.T_ref;  // x**1.5 as x*sqrt(x): within an ulp of pow, without its log/exp
     mu = b.mu_ref * (x * sqrt(x)) * ((b.T_ref + b.S_ref) / (T + b.S_ref));
     b.mu[c] = mu;
@@ -457,10 +480,10 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   if constexpr (NG == 6 || NG == 7) {
   double tk = b.qp[5 * b.nc + c], tw = b.qp[6 * b.nc + c];
   double mut, F1;
-  sst_mut_f1<S2003>(rho, tk, tw, b.dist[c], mu, gg, mut, F1);
+  sst_mut_f1<S2003>(rho, tk, tw, dist, mu, gg, mut, F1);
   if constexpr (NG == 7) {
     const long cl = ci(b, b.imx, b.jmx, b.kmx);
-    F1 = lctm_f1(F1, b.qp[cl], b.qp[5 * b.nc + cl], b.dist[c], mu);
+    F1 = lctm_f1(F1, b.qp[cl], b.qp[5 * b.nc + cl], dist, mu);
   }
   if (keep_m) {
     b.mut[c] = mut;
@@ -471,12 +494,12 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
     double S_k, S_w;
     if constexpr (NG == 7) {
       double S_gm;
-      lctm_source<S2003>(rho, tk, tw, b.qp[7 * b.nc + c], mut, F1, mu, b.dist[c], b.dvdy[c], vol, gg, S_k, S_w,
+      lctm_source<S2003>(rho, tk, tw, b.qp[7 * b.nc + c], mut, F1, mu, dist, b.dvdy[c], vol, gg, S_k, S_w,
                          S_gm);
       b.src[2 * b.nres + ri(b, i, j, k)] = S_gm;
     } else if constexpr (BC) {
       const double u = b.qp[b.nc + c], v = b.qp[2 * b.nc + c], w = b.qp[3 * b.nc + c];
-      sst_bc_source(b, rho, sqrt(u * u + v * v + w * w), tk, tw, mut, F1, mu, b.dist[c], vol, gg, S_k, S_w);
+      sst_bc_source(b, rho, sqrt(u * u + v * v + w * w), tk, tw, mut, F1, mu, dist, vol, gg, S_k, S_w);
     } else {
       sst_source<S2003>(rho, tk, tw, mut, F1, vol, gg, S_k, S_w);
     }
@@ -493,26 +516,20 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
     ghost_gradients<NG>(b, i, j, k, vol, gg, mut, 0.0);
     // the density gradient over the face sums rho_neighbour + rho
     const double *q0 = b.qp;
-    double rf[6] = {q0[c - si] + rho, q0[c - sj] + rho, q0[c - sk] + rho,
-                    q0[c + si] + rho, q0[c + sj] + rho, q0[c + sk] + rho};
     double grho[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       // the k-face normal of the lower k face is (nx, nx, nx)
-      double nk0 = n[0][2];
-      double g = -(rf[0] * n[d][0] * Ai0);
-      g = g - rf[1] * n[d][1] * Aj0;
-      g = g - rf[2] * nk0 * Ak0;
-      g = g + rf[3] * n[d][3] * Ai1;
-      g = g + rf[4] * n[d][4] * Aj1;
-      g = g + rf[5] * n[d][5] * Ak1;
-      grho[d] = g / (2.0 * vol);
+      double g = 0.0;
+#pragma unroll
+      for (int f = 0; f < 6; ++f) g = g + (q0[c + st[f + 1]] + rho) * m[f == 2 ? 0 : d][f];
+      grho[d] = g;
     }
     if constexpr (BC) {
       const double u = b.qp[b.nc + c], v = b.qp[2 * b.nc + c], w = b.qp[3 * b.nc + c];
-      b.src[ri(b, i, j, k)] = sa_bc_source(b, rho, sqrt(u * u + v * v + w * w), tv, mu, b.dist[c], vol, gg, grho);
+      b.src[ri(b, i, j, k)] = sa_bc_source(b, rho, sqrt(u * u + v * v + w * w), tv, mu, dist, vol, gg, grho);
     } else {
-      b.src[ri(b, i, j, k)] = sa_source(rho, tv, mu, b.dist[c], vol, gg, grho);
+      b.src[ri(b, i, j, k)] = sa_source(rho, tv, mu, dist, vol, gg, grho);
     }
   }
   }
