@@ -470,7 +470,10 @@ int launch_update(fest_handle *h, double TF, double SF, int flags) {
   dim3 g, t;
   box(b.imx - 1, b.jmx - 1, b.kmx - 1, g, t, b.xcd_remap);
   KgScope ts(h, KG_UPDATE);
-  hipLaunchKernelGGL(k_update, g, t, 0, h->stream, b, TF, SF, flags);
+  if (b.nv == 8) hipLaunchKernelGGL(k_update<8>, g, t, 0, h->stream, b, TF, SF, flags);
+  else if (b.nv == 7) hipLaunchKernelGGL(k_update<7>, g, t, 0, h->stream, b, TF, SF, flags);
+  else if (b.nv == 6) hipLaunchKernelGGL(k_update<6>, g, t, 0, h->stream, b, TF, SF, flags);
+  else hipLaunchKernelGGL(k_update<5>, g, t, 0, h->stream, b, TF, SF, flags);
   LAUNCHCHK(h);
   return 0;
 }
@@ -1584,7 +1587,10 @@ int run_group_op_batched(fest_group *g, const StepOp &op, int current_iter) {
       }
       break;
     case OP_DT: KM(PH_DT, km_dt, dim3(256)); break;
-    case OP_UPDATE: KM(PH_UPDATE, km_update, dim3(256), op.a, op.c, op.flags); break;
+    case OP_UPDATE:
+      if (b0.nv == 7) KM(PH_UPDATE, km_update<7>, dim3(256), op.a, op.c, op.flags);
+      else KM(PH_UPDATE, km_update<5>, dim3(256), op.a, op.c, op.flags);
+      break;
     default:
       for (fest_handle *h : g->blocks)
         if ((rc = run_op(h, op, current_iter))) return gfail(g, rc, "%s", h->err.c_str());

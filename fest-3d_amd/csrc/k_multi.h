@@ -38,9 +38,10 @@ __global__ void __launch_bounds__(256) km_dt(const Blk *__restrict__ blks, const
                                              int n) {
   FEST_WALK(k_dt_b(b, wg))
 }
+template <int NV>
 __global__ void __launch_bounds__(256) km_update(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
                                                  int n, double TF, double SF, int flags) {
-  FEST_WALK(k_update_b(b, wg, TF, SF, flags))
+  FEST_WALK(k_update_b<NV>(b, wg, TF, SF, flags))
 }
 __global__ void __launch_bounds__(256) km_to_f32(const Blk *__restrict__ blks, const WorkItem *__restrict__ items,
                                                  int n) {
