@@ -233,9 +233,13 @@ struct FaceMath {
   template <int RECON, typename Q>
   static __device__ __forceinline__ void face_states(const Blk &b, int d, int n, int N, int l, const Q *u,
                                                      long s, const Aux &ax, T &L, T &R) {
-    constexpr int recon = RECON;
     // cell n-3+m, read where it is used
-    auto w = [u, s](int m) { return T(u[(long)(m - 3) * s]); };
+    face_states_of<RECON>(b, d, n, N, l, [u, s](int m) { return T(u[(long)(m - 3) * s]); }, ax, L, R);
+  }
+  template <int RECON, typename W>
+  static __device__ __forceinline__ void face_states_of(const Blk &b, int d, int n, int N, int l, const W &w,
+                                                        const Aux &ax, T &L, T &R) {
+    constexpr int recon = RECON;
     const int sw = (l >= 5) ? b.tlim[d] : b.lim[d];
     const int minbc = b.bc[2 * d], maxbc = b.bc[2 * d + 1];
     const bool on = recon != 0;
@@ -539,7 +543,10 @@ struct FaceMath {
   // 128 (SST, WENO5) take 1205 -> 1090 us, of 384 x 192 x 128 (PPM) 2630 ->
   // 2380 us; two or three variables ahead 1130 us, the gradients asked for
   // before the inviscid flux 1175 us and up, with spills.  4.3 GB pass at 4.0
-  // TB/s then.  FP32, whose registers suffice, is left to the compiler.
+  // TB/s then.  FP32 takes the stencils ahead too (256 x 128 x 128 760 -> 682 us,
+  // 24 blocks of 1.1 M cells, MUSCL, 163 -> 145 us; two variables ahead the
+  // same); its viscous inputs fit the registers in the compiler's order (690 us
+  // in this one).
   static __device__ __forceinline__ void fence() {
     if constexpr (std::is_same<T, double>::value) __builtin_amdgcn_sched_barrier(0);
   }
@@ -695,7 +702,8 @@ __host__ __device__ inline long flux_i_span(const Blk &b) {
   return (b.imx + 2) + (long)(b.jmx + 1) * b.pi - flux_i_first(b) + 1;
 }
 
-// stencils that are on their way while a variable is reconstructed (see fence)
+// stencils of the j and k sweeps that are on their way while a variable is
+// reconstructed (see fence)
 constexpr int AHEAD = 1;
 template <int D, int NV, int RECON, bool FLAT, typename T>
 __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int store_csnd) {
@@ -767,13 +775,14 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int
     // it (439 -> 466 us; 97 x 61 x 45, all three, 98 -> 103 us), and FP32 keeps
     // the one form its results are defined by.
     constexpr bool split = D != 0 && std::is_same<T, double>::value;
-    if (!split || M::template edge_face<RECON>(b, D, n, N)) {
+    if constexpr (D == 0) {
 #pragma unroll
-      for (int l = 0; l < nv; ++l) {
-        if constexpr (D == 0)
-          M::template face_states<RECON>(b, D, n, N, l, lds_row + l * (FLUX_I_SPAN + 5), 1, ax, qL[l], qR[l]);
-        else M::template face_states<RECON>(b, D, n, N, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
-      }
+      for (int l = 0; l < nv; ++l)
+        M::template face_states<RECON>(b, D, n, N, l, lds_row + l * (FLUX_I_SPAN + 5), 1, ax, qL[l], qR[l]);
+    } else if (split && M::template edge_face<RECON>(b, D, n, N)) {
+#pragma unroll
+      for (int l = 0; l < nv; ++l)
+        M::template face_states<RECON>(b, D, n, N, l, qsrc + (long)l * b.nc + c, s, ax, qL[l], qR[l]);
     } else {
       T w[AHEAD + 1][6];
 #pragma unroll
@@ -782,8 +791,10 @@ __device__ __forceinline__ void k_flux_b(const Blk &b, const Wg &wg, int ti, int
       for (int l = 0; l < nv; ++l) {
         if (l + AHEAD < nv)
           M::template stencil<RECON>(qsrc + (long)(l + AHEAD) * b.nc + c, s, w[(l + AHEAD) % (AHEAD + 1)]);
-        M::fence();
-        M::template inner_states<RECON>(b, D, l, w[l % (AHEAD + 1)], ax, qL[l], qR[l]);
+        __builtin_amdgcn_sched_barrier(0);
+        const T(&u)[6] = w[l % (AHEAD + 1)];
+        if constexpr (split) M::template inner_states<RECON>(b, D, l, u, ax, qL[l], qR[l]);
+        else M::template face_states_of<RECON>(b, D, n, N, l, [&u](int m) { return u[m]; }, ax, qL[l], qR[l]);
       }
     }
     if (store_csnd) csf = T(0.5) * (tsqrt(T(b.gm) * qL[4] / qL[0]) + tsqrt(T(b.gm) * qR[4] / qR[0]));
