@@ -65,7 +65,15 @@ struct Dual {
   friend __device__ __forceinline__ bool operator>=(const Dual &a, const Dual &b) { return a.v >= b.v; }
 
   // the face arithmetic's helpers (blk.h, k_flux.h) for dual arguments
-  friend __device__ __forceinline__ Dual tdiv(const Dual &a, const Dual &b) { return a / b; }
+  // as operator/ with qdiv, for the quotients whose divisor is never zero
+  friend __device__ __forceinline__ Dual tdiv(const Dual &a, const Dual &b) {
+    Dual r;
+    const double ib = qdiv(1.0, b.v);
+    r.v = a.v * ib;
+#pragma unroll
+    for (int k = 0; k < K; ++k) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib;
+    return r;
+  }
   friend __device__ __forceinline__ Dual xdiv(const Dual &a, const Dual &b) { return a / b; }
   friend __device__ __forceinline__ Dual tsqrt(const Dual &a) {
     Dual r;

@@ -10,23 +10,12 @@ namespace {
 
 inline unsigned blocks(long n) { return (unsigned)((n + 255) / 256); }
 
-template <int D, int RECON>
-void vjp_dir_t(const Blk &b, hipStream_t st, const double *barR, double *c, double *mbar) {
-  const long nf = b.nfl[D];
-  double *fbar = c + (long)VJP_PER_FACE * nf;  // bar qL, bar qR after the contributions
-  hipLaunchKernelGGL((k_vjp_flux<D, RECON>), dim3(blocks(nf)), dim3(256), 0, st, b, barR, fbar, mbar);
-  double *pbc = fbar + 10 * nf;  // the pressure-based switch's pressure contributions, when it is on
-  hipLaunchKernelGGL((k_vjp_recon<D, RECON>), dim3(blocks(5 * nf)), dim3(256), 0, st, b, fbar, c, pbc);
-}
-template <int D>
-void vjp_dir(const Blk &b, hipStream_t st, const double *barR, double *c, double *mbar) {
-  switch (b.recon) {
-    case 0: vjp_dir_t<D, 0>(b, st, barR, c, mbar); break;
-    case 1: vjp_dir_t<D, 1>(b, st, barR, c, mbar); break;
-    case 2: vjp_dir_t<D, 2>(b, st, barR, c, mbar); break;
-    case 3: vjp_dir_t<D, 3>(b, st, barR, c, mbar); break;
-    default: vjp_dir_t<D, 4>(b, st, barR, c, mbar); break;
-  }
+template <int RECON>
+void vjp_faces(const Blk &b, hipStream_t st, const double *barR, const VjpDirs &v) {
+  const unsigned f0 = blocks(b.nfl[0]), f1 = blocks(b.nfl[1]), f2 = blocks(b.nfl[2]);
+  hipLaunchKernelGGL(k_vjp_flux<RECON>, dim3(f0 + f1 + f2), dim3(256), 0, st, b, barR, v, f0, f1);
+  const unsigned r0 = 5 * f0, r1 = 5 * f1, r2 = 5 * f2;
+  hipLaunchKernelGGL(k_vjp_recon<RECON>, dim3(r0 + r1 + r2), dim3(256), 0, st, b, v, r0, r1);
 }
 
 }  // namespace
@@ -38,9 +27,18 @@ long vjp_contrib_len(const Blk &b, int d) {
 
 void launch_vjp(const Blk &b, hipStream_t st, const double *barR, double *const contrib[3], double *bar,
                 const VjpNodes &nodes, const VjpVisc &visc) {
-  vjp_dir<0>(b, st, barR, contrib[0], nodes.mbar[0]);
-  vjp_dir<1>(b, st, barR, contrib[1], nodes.mbar[1]);
-  vjp_dir<2>(b, st, barR, contrib[2], nodes.mbar[2]);
+  VjpDirs v;
+  for (int d = 0; d < 3; ++d) {
+    v.c[d] = contrib[d];
+    v.mbar[d] = nodes.mbar[d];
+  }
+  switch (b.recon) {
+    case 0: vjp_faces<0>(b, st, barR, v); break;
+    case 1: vjp_faces<1>(b, st, barR, v); break;
+    case 2: vjp_faces<2>(b, st, barR, v); break;
+    case 3: vjp_faces<3>(b, st, barR, v); break;
+    default: vjp_faces<4>(b, st, barR, v); break;
+  }
   hipLaunchKernelGGL(k_vjp_gather, dim3(blocks(b.nc)), dim3(256), 0, st, b, contrib[0], contrib[1], contrib[2], bar);
   if (visc.bt) {
     hipLaunchKernelGGL(k_vjp_visc<0>, dim3(blocks(b.nfl[0])), dim3(256), 0, st, b, barR, contrib[0]);
@@ -56,11 +54,14 @@ void launch_vjp(const Blk &b, hipStream_t st, const double *barR, double *const 
     hipLaunchKernelGGL(k_vjp_grad, dim3(blocks(b.nc)), dim3(256), 0, st, b, visc.gb, visc.bt, bar);
   }
   // the k faces of a 2-D grid (one cell in k) feed no flux
-  for (int face = b.kmx == 2 ? 3 : 5; face >= 0; --face) {
+  for (int face = b.kmx == 2 ? 3 : 5; face >= 0;) {
     const int na = face_na(b, face), nb = face_nb(b, face);
+    const int cells = (face < 2 ? b.imx : face < 4 ? b.jmx : b.kmx) - 1;
+    const unsigned n = (face & 1) && cells >= 8 ? 2 : 1;
     double *gface = face == 3 ? nodes.g3 : face == 5 ? nodes.g5 : nullptr;
-    hipLaunchKernelGGL(k_vjp_bc, dim3(blocks(na - 1), (unsigned)(nb - 1)), dim3(256), 0, st, b, face, bar,
+    hipLaunchKernelGGL(k_vjp_bc, dim3(blocks(na - 1), (unsigned)(nb - 1), n), dim3(256), 0, st, b, face, bar,
                        nodes.mbar[0], nodes.mbar[1], nodes.mbar[2], gface);
+    face -= (int)n;
   }
   if (!nodes.bar_nodes) return;
   // the metric adjoints to the face diagonals (into the contribution

@@ -122,3 +122,29 @@ def test_norm_sums(ni, nj, nk, turb):
     exact = abs(float(sum(e.sum() for e in ends)))
     mag = float(sum(abs(e).sum() for e in ends))
     assert abs(norms[0] - exact) <= (m * 2.0**-53 + 1e-14) * mag
+
+
+@pytest.mark.parametrize("turb", ["none", "sst", "sa"])
+@pytest.mark.parametrize("ni,nj,nk", [(5, 4, 1), (64, 3, 2), (65, 5, 3), (3, 9, 1)])
+def test_gradients_next_to_boundaries(ni, nj, nk, turb):
+    """Gradients and mu_t of interior and first ghost cells where a direction
+    has one cell (both its faces belong to it), two or three, and rows that
+    end at and past a wave."""
+    if turb == "none":
+        case, nodes, q = C.laminar_box(ni, nj, nk)
+        nodes = C.cartesian_nodes(case, warp=0.03)
+        case = dataclasses.replace(case, bc_id=(-8, -4, -5, -5, -6, -6), fix_p=(case.p_inf,) * 6)
+    else:
+        case, nodes, q = C.sst_bump(ni, nj, nk, turb=turb, recon="muscl", first=0.02)
+        case = dataclasses.replace(case, bc_id=case.bc_id[:4] + (-6, -6))
+    print("gradients", ni, nj, nk, turb, flush=True)
+    g, o = pair(case, nodes, q, turb != "none")
+    assert o.residual(3) == 0
+    g.residual(3)
+    out = g.download("grads", "mut", "residue")
+    for d, n in enumerate(("gx", "gy", "gz")):
+        assert relerr(out["grads"][d], o.arr(n)) <= TOL, n
+    if turb != "none":
+        inner = (slice(2, -2),) * 3
+        assert relerr(out["mut"][inner], o.arr("mut")[inner]) <= TOL
+    assert relerr(out["residue"], o.arr("res")) <= TOL
