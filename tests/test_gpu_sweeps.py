@@ -125,10 +125,10 @@ def test_norm_sums(ni, nj, nk, turb):
 
 
 @pytest.mark.parametrize("turb", ["none", "sst", "sa"])
-@pytest.mark.parametrize("ni,nj,nk", [(5, 4, 1), (64, 3, 2), (65, 5, 3), (3, 9, 1)])
+@pytest.mark.parametrize("ni,nj,nk", [(5, 4, 1), (64, 3, 3), (65, 5, 4), (3, 9, 1)])
 def test_gradients_next_to_boundaries(ni, nj, nk, turb):
     """Gradients and mu_t of interior and first ghost cells where a direction
-    has one cell (both its faces belong to it), two or three, and rows that
+    has one cell (both its faces belong to it), three or more, and rows that
     end at and past a wave."""
     if turb == "none":
         case, nodes, q = C.laminar_box(ni, nj, nk)
