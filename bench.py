@@ -24,8 +24,8 @@ ids).
 
 --time-accuracy implicit times the reference's LU-SGS integrator on the same
 workload instead: a step is one residual evaluation, the time step and the
-LU-SGS update (two sweeps of one launch per hyperplane i+j+k); the metric
-is cell-implicit-steps per second and the CPU baseline times the oracle's
+LU-SGS update (two sweeps of one launch each); the metric is
+cell-implicit-steps per second and the CPU baseline times the oracle's
 implicit step.
 """
 import argparse
@@ -44,7 +44,7 @@ def measured_traffic(case, group):
     """HBM bytes per launch of `group`'s FP64 kernel from the committed
     counter summary profiles/hbm_traffic_<workload>_<size>.md (its table rows
     read `| group | kernel | fetch B | write B | traffic B |`; the FP32 face
-    kernels, `k_flux<..., float>`, have rows of their own), else None."""
+    kernels, `..., float>`, have rows of their own), else None."""
     path = os.path.join(PROFILES, f"hbm_traffic_{case.name}.md")
     if not os.path.exists(path):
         return None

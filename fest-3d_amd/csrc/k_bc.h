@@ -1,9 +1,10 @@
-// k_bc.h -- ghost-cell boundary conditions (one launch per block face, in
-// the reference's face order imin, imax, jmin, jmax, kmin, kmax), then the
-// edge/corner averages.  src/boundary/bc_primitive.f90:55-227 and the
-// routines it calls; every face kernel gives one thread a column of three
-// ghost cells, which only reads its own column, so the per-face passes keep
-// the reference's sequential semantics.  The bodies and helpers are here,
+// k_bc.h -- ghost-cell boundary conditions (faces in the reference's order
+// imin, imax, jmin, jmax, kmin, kmax, those that do not read each other's
+// ghosts in one launch), then the edge/corner averages.
+// src/boundary/bc_primitive.f90:55-227 and the routines it calls; every face
+// kernel gives one thread a column of three ghost cells, which only reads its
+// own column, so the passes keep the reference's sequential
+// semantics.  The bodies and helpers are here,
 // their per-block kernels in k_bc_kernels.h (one translation unit).
 #pragma once
 // ghost cells and geometry keep the reference's unfused operation order

@@ -11,7 +11,7 @@
 // on qR (the 5 x 10 flux Jacobian, contracted at once with the face's
 // adjoint flux barF = barR(n-1) - barR(n) into bar qL, bar qR);
 // k_vjp_recon, one thread per face and variable, differentiates that
-// variable's reconstruction with tangents on its six stencil values.
+// variable's reconstruction with tangents on the stencil values it reads.
 // k_vjp_gather sums, for every cell, the contributions of the faces whose
 // stencils hold it (in a fixed order: deterministic), and k_vjp_bc moves the
 // adjoints of ghost cells onto the interior cells the ghost rules read.

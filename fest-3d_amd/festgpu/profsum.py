@@ -29,19 +29,18 @@ from . import roofline as R
 
 
 GROUPS = [  # (substring of the demangled kernel name, kernel group)
-    ("k_flux<0", "flux_i"), ("k_flux<1", "flux_j"), ("k_flux<2", "flux_k"),
-    ("k_grad<", "grad"), ("k_grad_bc", "grad_bc"), ("k_mut_ghost_tp", "grad_bc"), ("k_update", "update"),
+    ("k_sweeps<", "flux"),  # the three directions in one launch
+    ("k_grad<", "grad"), ("k_mut_ghost_tp", "grad_bc"), ("k_update", "update"),
     ("k_bc_face", "bc_face"), ("k_bc_edges", "bc_edges"), ("k_step_begin", "step_begin"),
     ("k_dt_min", "time_step"), ("k_dt_fill", "time_step"), ("k_dt", "time_step"),
-    ("k_norm", "resnorm"), ("k_node_dist", "setup"), ("k_cell_dist", "setup"), ("k_cells", "setup"),
+    ("k_norm", "resnorm"), ("k_report", "resnorm"), ("k_node_dist", "setup"), ("k_cell_dist", "setup"), ("k_cells", "setup"),
     ("k_face_metrics", "setup"), ("k_ghost_nodes", "setup"), ("k_fill", "setup"),
-    ("k_lusgs_sweep", "lusgs_sweep"), ("k_lusgs_prep", "lusgs_diag"),
+    ("k_lusgs_march", "lusgs_sweep"), ("k_lusgs_empty", "setup"), ("k_lusgs_prep", "lusgs_diag"),
     ("k_to_skew", "lusgs_diag"), ("k_lusgs_apply", "lusgs_apply"), ("k_exchange", "exchange"),
     ("k_kkl_source", "kkl_source"), ("k_to_f32", "f32_copy"), ("k_g32_widen", "f32_copy"),
     ("k_vjp_", "vjp"),
     # batched group steps: one launch per phase over all blocks
-    ("km_flux<0", "flux_i"), ("km_flux<1", "flux_j"), ("km_flux<2", "flux_k"), ("km_grad<", "grad"),
-    ("km_grad_bc", "grad_bc"), ("km_update", "update"), ("km_bc_face", "bc_face"), ("km_bc_edges", "bc_edges"),
+    ("km_sweeps<", "flux"), ("km_grad<", "grad"), ("km_update", "update"), ("km_bc_face", "bc_face"), ("km_bc_edges", "bc_edges"),
     ("km_step_begin", "step_begin"), ("km_dt", "time_step"), ("km_to_f32", "f32_copy"),
 ]
 
@@ -54,7 +53,7 @@ def group_of(name):
 
 
 def short(name):
-    """fest::k_flux<0>(fest::Blk, int) -> k_flux<0>"""
+    """fest::k_update<7>(fest::Blk, double, double, int) -> k_update<7>"""
     n = name.split("(")[0]
     for pre in ("void ", "fest::"):
         n = n.replace(pre, "")

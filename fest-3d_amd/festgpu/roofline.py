@@ -6,7 +6,8 @@ from cache), FP64 throughout.  Face arrays are counted per face, cell arrays
 per cell of the launch's index box.  The numbers follow the kernels in
 fest-3d_amd/csrc:
 
-  flux_i/j/k (k_flux<D>, one thread per face of direction D):
+  flux_i/j/k (k_sweeps run for one direction D, as timed runs do; one thread
+  per face of direction D):
     read  q (n_var planes), the face's A,nx,ny,nz (4), both cell centres
           (3, one per cell), the cell gradients (3 x n_grad), mu (+ mu_t, F1
           with SST)
@@ -24,22 +25,22 @@ fest-3d_amd/csrc:
           cell), the RK base state (n_var), dt, volume, the R accumulator
           (stages 2-4), the SST source (2), F1 and omega (SST)
     write q (n_var), the R accumulator (stages 1-3), the residue (stage 4)
-  lusgs_sweep (k_lusgs_sweep, the LU-SGS update of the 'implicit' step: one
-    launch per hyperplane i+j+k = s, 2 (ni+nj+nk-2) launches a step, which
-    the engine's event timer brackets as one; priced per bracket, i.e. both
-    sweeps over every interior cell), per interior cell and sweep, from the
-    hyperplane-major storage:
-    read  q (n_var), three faces x {A,nx,ny,nz}, volume, mu, mu_t, F1, three
-          radii, three Old fluxes (3 x n_var), the diagonal (1, or 3 with
-          SST), the right-hand side (residue or own value, n_var), the
-          neighbours' sweep values (n_var, each value once)
-    write the sweep value (n_var)
+  lusgs_sweep (k_lusgs_march, the LU-SGS update of the 'implicit' step: one
+    launch a sweep, two a step, which the engine's event timer brackets as
+    one; priced per bracket, i.e. both sweeps over every interior cell), per
+    interior cell and sweep, from the hyperplane-major storage, whose values
+    are kept in pairs (p = ceil(n_var / 2)):
+    read  the state, the right-hand side and, backward, the cell's own
+          forward value (p pairs each), the diagonal (1 pair, SST 2), three
+          faces x {A,nx,ny,nz, the viscous factors (2, turbulent 4), radius}
+          in 4 or 5 pairs
+    write the sweep value (p pairs)
   lusgs_diag (k_to_skew + k_lusgs_prep, once a step), per interior cell:
-    the copies of q, mu, mu_t, F1 and the residue into hyperplane-major
-    storage (read + write, 2 x (2 n_var + 3)); the prep's stencil reads (q,
-    six faces x 4 metrics counted once a face, volume, mu, mu_t, F1, centres,
-    dt: n_var + 12 + 8) and writes (three radii, six Old fluxes, diagonal:
-    3 + 6 n_var + 1 or 3)
+    the copy of q into hyperplane-major storage (read + write, 2 n_var); the
+    prep's stencil reads (q and residue, six faces x 4 metrics counted once a
+    face, volume, mu, mu_t, F1, centres, dt: 2 n_var + 12 + 8) and writes (two
+    right-hand sides, three radii, three faces' viscous factors, diagonal:
+    2 n_var + 3 + 6 or 12 + 1 or 3)
   lusgs_apply (k_lusgs_apply): read q and the sweep value, write q (3 n_var)
 """
 
@@ -48,11 +49,6 @@ W = 8  # bytes per FP64 value
 
 def _ngrad(case):
     return 6 if case.sst_family else 4
-
-
-def lusgs_launches(case):
-    """Hyperplane launches of the two LU-SGS sweeps of one step."""
-    return 2 * ((case.imx - 1) + (case.jmx - 1) + (case.kmx - 1) - 2)
 
 
 def launch_items(case, group):
@@ -94,12 +90,12 @@ def bytes_per_item(case, group):
         acc = (nv + 2 * nv + 2 * nv + 2 * nv) / 4.0  # R: write; read+write x2; read + residue write
         return W * (base + acc)
     ndg = 3 if sst else 1
+    pairs, nvis = (nv + 1) // 2, 2 if nv == 5 else 4
     if group == "lusgs_sweep":
-        reads = nv + 12 + 4 + 3 + 3 * nv + ndg + nv + nv
-        return W * (reads + nv)
+        reads = 2.5 * pairs + (ndg + 1) // 2 + 3 * (3 + nvis // 2)
+        return 2 * W * (reads + pairs)
     if group == "lusgs_diag":
-        copies = 2 * (2 * nv + 3)
-        return W * (copies + (nv + 12 + 8) + (3 + 6 * nv + ndg))
+        return W * (2 * nv + (2 * nv + 12 + 8) + (2 * nv + 3 + 3 * nvis + ndg))
     if group == "lusgs_apply":
         return W * 3 * nv
     return None
