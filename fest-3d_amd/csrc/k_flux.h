@@ -542,7 +542,7 @@ struct FaceMath {
   // viscous flux's inputs one gradient ahead, all three sweeps of 256 x 128 x
   // 128 (SST, WENO5) take 1205 -> 1090 us, of 384 x 192 x 128 (PPM) 2630 ->
   // 2380 us; two or three variables ahead 1130 us, the gradients asked for
-  // before the inviscid flux 1175 us and up, with spills.  4.3 GB pass at 4.0
+  // before the inviscid flux 1175 us and up, with spills.  4.0 GB pass at 3.7
   // TB/s then.  FP32 takes the stencils ahead too (256 x 128 x 128 760 -> 682 us,
   // 24 blocks of 1.1 M cells, MUSCL, 163 -> 145 us; two variables ahead the
   // same); its viscous inputs fit the registers in the compiler's order (690 us

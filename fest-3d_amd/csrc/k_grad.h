@@ -374,7 +374,7 @@ __device__ __forceinline__ void k_grad_b(const Blk &b, const Wg &wg) {
   // sum: loads and stores retire in order, so a load behind a store waits for
   // it too.  With each variable loaded, summed and stored in turn the waits of
   // a whole memory latency were one a variable: 256
-  // x 128 x 128 (SST) 460 -> 435 us (1.7 GB, 3.9 TB/s), 128 x 96 x 64 (SA) 99
+  // x 128 x 128 (SST) 460 -> 435 us (1.6 GB, 3.7 TB/s), 128 x 96 x 64 (SA) 99
   // -> 83 us, 97 x 61 x 45 44 -> 40 us, 64 x 64 x 4 (laminar) 10.8 -> 9.0 us.
   // It takes 142 registers (SST), 3 waves a SIMD; held to 4 it spills (479 us).
   V w[2][7];

@@ -40,7 +40,7 @@ __device__ __forceinline__ double sspd(const Blk &b, int d, long o) { return b.c
 // Memory bound.  The face metrics, speeds and velocities are asked for at once,
 // the centres with them, and the viscous limit's six quotients serve mu and
 // mu_t alike (one each, times two, in turn before): 256 x 128 x 128 256 -> 234
-// us (0.87 GB, 3.7 TB/s), 24 blocks of 1.1 M cells 75 -> 55, 128 x 96 x 64 49 -> 42.
+// us (1.35 GB, 5.8 TB/s), 24 blocks of 1.1 M cells 75 -> 55, 128 x 96 x 64 49 -> 42.
 __device__ __forceinline__ void k_dt_b(const Blk &b, const Wg &wg) {
   int i, j;
   bool active = flat_ij(b.imx - 1, b.jmx - 1, i, j, (int)wg.x);
