@@ -322,7 +322,10 @@ __device__ __forceinline__ long vjp_rface(const Blk &b, int face, int a, int bb)
 // -8, -11) add their normals' adjoints there; the slip wall's ghost-row I
 // face of the j and k max faces goes to gface[c][(a-1) + (na-1)(bb-1)].
 // A direction's two faces go in one launch (grid z, the higher first) where
-// they have 8 cells between them: a ghost column reads up to layer 4.  Six
+// neither adds to cells that the other adds to: with 8 cells between them a
+// ghost column reads up to layer 4 on its own side, but a periodic face reads
+// the three layers next to the other one, which only another periodic face
+// leaves alone (a direction with one periodic face takes two launches).  Six
 // launches of 12 us each, so three.
 __global__ void __launch_bounds__(256) k_vjp_bc(Blk b, int face0, double *bar, double *mb0, double *mb1, double *mb2,
                                                 double *gface0) {

@@ -57,7 +57,8 @@ void launch_vjp(const Blk &b, hipStream_t st, const double *barR, double *const 
   for (int face = b.kmx == 2 ? 3 : 5; face >= 0;) {
     const int na = face_na(b, face), nb = face_nb(b, face);
     const int cells = (face < 2 ? b.imx : face < 4 ? b.jmx : b.kmx) - 1;
-    const unsigned n = (face & 1) && cells >= 8 ? 2 : 1;
+    const bool across = (b.bc[face & ~1] == -9) != (b.bc[face | 1] == -9);
+    const unsigned n = (face & 1) && cells >= 8 && !across ? 2 : 1;
     double *gface = face == 3 ? nodes.g3 : face == 5 ? nodes.g5 : nullptr;
     hipLaunchKernelGGL(k_vjp_bc, dim3(blocks(na - 1), (unsigned)(nb - 1), n), dim3(256), 0, st, b, face, bar,
                        nodes.mbar[0], nodes.mbar[1], nodes.mbar[2], gface);
