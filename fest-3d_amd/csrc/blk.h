@@ -99,6 +99,17 @@ __host__ __device__ inline long ci(const Blk &b, int i, int j, int k) {
 __host__ __device__ inline long fi(const Blk &b, int d, int i, int j, int k) {
   return (long)(i + 2) + (long)b.fpi[d] * ((long)(j + 2) + (long)b.fpj[d] * (long)(k + 2));
 }
+// The metrics that the ghost-gradient rule reads for face (i, j, k) of
+// direction d.  The reference passes Jfaces/Kfaces to a dummy declared with the
+// I-face extents, so the J/K metrics are read at the I-face linear offset
+// (src/gradients.f90:523-588 calling :591); that is reproduced.  In a block far
+// longer along k (or j) than along i that offset passes the end of the J or K
+// arrays, where the reference reads whatever memory follows: there the face's
+// own metrics are taken.
+__device__ __forceinline__ long ghost_metrics(const Blk &b, int d, int i, int j, int k) {
+  const long o = fi(b, 0, i, j, k);
+  return o < b.nfc[d] ? o : fi(b, d, i, j, k);
+}
 // F/G/H index of direction d
 __host__ __device__ inline long fli(const Blk &b, int d, int i, int j, int k) {
   return (long)(i - 1) + (long)b.nfi[d] * ((long)(j - 1) + (long)b.nfj[d] * (long)(k - 1));

@@ -267,9 +267,7 @@ __device__ __forceinline__ bool visc_rule(const Blk &b, int id) {
 // own gradients gg, mu_t and F1 are all the rules need, so its thread writes
 // them: with a pass of its own over the six faces a stage's gradients took
 // 400 + 83 us at 256x128x128 (SST) and 29 + 22 us at 97x61x45, together 435 and
-// 40.  The reference passes Jfaces/Kfaces to a dummy declared with the I-face extents, so the J/K metrics are read at the
-// I-face linear offset (src/gradients.f90:523-588 calling :591); that is
-// reproduced.
+// 40.
 template <int NG>
 __device__ __forceinline__ void ghost_gradients(const Blk &b, int i, int j, int k, double vol,
                                                 const double (&gg)[NG][3], double mut, double F1) {
@@ -286,7 +284,7 @@ __device__ __forceinline__ void ghost_gradients(const Blk &b, int i, int j, int 
       if (id >= 0) continue;
       const double Tw = hi ? b.fix[FX_TWALL][2 * d + 1] : b.fix[FX_TWALL][2 * d];
       const int fp = hi ? N : 1, g = hi ? N : 0;  // the face and its first ghost layer
-      const long fo = d == 0 ? fi(b, 0, fp, j, k) : d == 1 ? fi(b, 0, i, fp, k) : fi(b, 0, i, j, fp);
+      const long fo = d == 0 ? fi(b, 0, fp, j, k) : d == 1 ? ghost_metrics(b, 1, i, fp, k) : ghost_metrics(b, 2, i, j, fp);
       const long cG = d == 0 ? ci(b, g, j, k) : d == 1 ? ci(b, i, g, k) : ci(b, i, j, g);
       const long gG = d == 0 ? gri(b, g, j, k) : d == 1 ? gri(b, i, g, k) : gri(b, i, j, g);
       const double nx = b.fx[d][fo], ny = b.fy[d][fo], nz = b.fz[d][fo], A = b.fA[d][fo];

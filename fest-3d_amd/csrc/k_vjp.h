@@ -818,7 +818,7 @@ __global__ void __launch_bounds__(256) k_vjp_grad_bc(Blk b, int face, double *ba
   int Ii = fi_, Ij = fj_, Ik = fk_, Gi = fi_, Gj = fj_, Gk = fk_;
   if (hi) { if (d == 0) Ii--; else if (d == 1) Ij--; else Ik--; }
   else { if (d == 0) Gi--; else if (d == 1) Gj--; else Gk--; }
-  const long fo = fi(b, 0, fi_, fj_, fk_);  // the rule reads every direction's metrics at the I-face offset
+  const long fo = ghost_metrics(b, d, fi_, fj_, fk_);
   const double nx = b.fx[d][fo], ny = b.fy[d][fo], nz = b.fz[d][fo], A = b.fA[d][fo];
   const long cI = ci(b, Ii, Ij, Ik), cG = ci(b, Gi, Gj, Gk);
   const double vI = b.vol[cI];

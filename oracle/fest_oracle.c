@@ -1363,7 +1363,10 @@ static int gradient_G(orc *s, double *grad, const double *var, int dir) {
  * dummy with the I-face extents (-2:imx+3,-2:jmx+2,-2:kmx+2) and is called
  * with Jfaces and Kfaces too (gradients.f90:559,571,583,595); by sequence
  * association the J/K metrics are then read at the I-face linear offset.
- * That is reproduced here: every direction indexes its face arrays with IFI. */
+ * That is reproduced here: every direction indexes its face arrays with IFI.
+ * In a block far longer along k (or j) than along i that offset passes the end
+ * of the J or K arrays, where the reference reads whatever memory follows; the
+ * face's own metrics are taken there. */
 static void gradient_bc_face(orc *s, int face) {
   int d = face / 2, hi = face % 2;
   int id = s->c.bc_id[face];
@@ -1373,7 +1376,8 @@ static void gradient_bc_face(orc *s, int face) {
   const double *fx = s->a[d == 0 ? ORC_INX : d == 1 ? ORC_JNX : ORC_KNX];
   const double *fy = s->a[d == 0 ? ORC_INY : d == 1 ? ORC_JNY : ORC_KNY];
   const double *fz = s->a[d == 0 ? ORC_INZ : d == 1 ? ORC_JNZ : ORC_KNZ];
-  size_t (*gidx)(const orc *, int, int, int) = IFI;
+  size_t (*own)(const orc *, int, int, int) = d == 0 ? IFI : d == 1 ? JFI : KFI;
+  size_t nface = d == 0 ? s->nif : d == 1 ? s->njf : s->nkf;
   int n = d == 0 ? IMX : d == 1 ? JMX : KMX;
   int fpos = hi ? n : 1;
   int sig = hi ? -1 : 1;
@@ -1386,7 +1390,8 @@ static void gradient_bc_face(orc *s, int face) {
     int Ii = fi_, Ij = fj_, Ik = fk_, Gi = fi_, Gj = fj_, Gk = fk_;
     if (hi) { if (d == 0) Ii--; else if (d == 1) Ij--; else Ik--; }
     else { if (d == 0) Gi--; else if (d == 1) Gj--; else Gk--; }
-    size_t gf = gidx(s, fi_, fj_, fk_);
+    size_t gf = IFI(s, fi_, fj_, fk_);
+    if (gf >= nface) gf = own(s, fi_, fj_, fk_);
     double nx = fx[gf], ny = fy[gf], nz = fz[gf];
     double vI = vol[CI(s, Ii, Ij, Ik)];
     double c_x = fA[gf] * nx / vI, c_y = fA[gf] * ny / vI, c_z = fA[gf] * nz / vI;
