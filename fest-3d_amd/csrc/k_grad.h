@@ -557,7 +557,7 @@ __global__ void k_g32_widen(Blk b) {
 // A -11 face has no mu_t / F1 ghost rule (src/viscosity.f90:284-339,
 // 409-465 list -1..-9): its ghost cells keep the SST values
 // calculate_viscosity computes there, from the ghost gradients k_grad has
-// written.  Launched after it, only when an SST block has a -11 face.
+// written (the FP32 ones where only those are kept).  Launched after it, only when an SST block has a -11 face.
 __device__ __forceinline__ void k_mut_ghost_tp_b(const Blk &b, const Wg &wg) {
   int face = wg.z;
   int a = wg.x * blockDim.x + threadIdx.x + 1;
@@ -574,9 +574,9 @@ __device__ __forceinline__ void k_mut_ghost_tp_b(const Blk &b, const Wg &wg) {
   double gg[6][3];
 #pragma unroll
   for (int l = 0; l < 6; ++l) {
-    gg[l][0] = b.g[0][(long)l * b.ngr + gG];
-    gg[l][1] = b.g[1][(long)l * b.ngr + gG];
-    gg[l][2] = b.g[2][(long)l * b.ngr + gG];
+    const long o = (long)l * b.ngr + gG;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) gg[l][e] = b.g32only ? (double)b.g32[e][o] : b.g[e][o];
   }
   double mut, F1;
   double rho = b.qp[cG], tk = b.qp[5 * b.nc + cG], tw = b.qp[6 * b.nc + cG];
