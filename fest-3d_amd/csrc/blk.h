@@ -200,20 +200,23 @@ __device__ __forceinline__ double fmn(double a, double b) { return a < b ? a : b
 __device__ __forceinline__ double fsgn(double a, double b) { return copysign(fabs(a), b); }
 __device__ __forceinline__ double sqd(double x) { return x * x; }
 // The compiler's FP64 quotient: v_rcp_f64, two Newton steps, the quotient and
-// its remainder correction -- wrapped in v_div_scale, v_div_fmas and
-// v_div_fixup, which rescale operands near the ends of the exponent range.
-// The wrapper costs 3 of 11 instructions and runs every quotient of a thread
-// through VCC one after the other.  qdiv is the same sequence without it: the
-// same bits wherever b, 1/b and the quotient are normal numbers, as they are
-// for the face arithmetic's quotients (|b| from 1e-28, the WENO weights, to
-// 1e64).  Not for quotients that may be 0/0 or x/0: those take NaN here
-// (bmuscl_cell divides by plain differences and keeps a / b).
+// its remainder correction -- wrapped in v_div_scale and v_div_fmas, which
+// rescale operands near the ends of the exponent range and run every quotient
+// of a thread through VCC one after the other, and in v_div_fixup, which gives
+// x/0, x/Inf and their like.  qdiv leaves the first two out: the same bits
+// wherever b, 1/b and the quotient are normal numbers.  The face arithmetic's
+// and the LU-SGS sweeps' divisors are, or are 0 or Inf (a time step of 0 makes
+// the LU-SGS diagonal Inf, a cell without pressure a sound speed 0): the
+// widest are the WENO weights' sums, from eps^4 = 1e-24 to the 8th power of the
+// jump across a stencil (omega next to a wall jumps by 1e9 and more: 1e72;
+// 1e38 would be too much).  Not for quotients of plain differences, which may
+// be subnormal (bmuscl_cell keeps a / b).
 __device__ __forceinline__ double qdiv(double a, double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
   y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
   const double q = a * y;
-  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
 }
 // FP32 forms for the single-precision face arithmetic
 __device__ __forceinline__ float fmx(float a, float b) { return a > b ? a : b; }
