@@ -1,8 +1,8 @@
 """Summaries of rocprofv3 CSV output for the engine's kernels.
 
   python -m festgpu.profsum stats DIR
-      kernel table from the *_kernel_stats.csv under DIR (--kernel-trace
-      --stats --output-format csv): calls, average and total duration.
+      kernel table from the *_kernel_trace.csv under DIR (--kernel-trace
+      --output-format csv): calls, average and total duration.
   python -m festgpu.profsum sq DIR [DIR ...]
       per-kernel VALU and wait figures from --pmc runs with SQ_WAVES,
       SQ_INSTS_VALU, SQ_WAVE_CYCLES, SQ_WAIT_INST_ANY, SQ_INSTS_VMEM_RD,
@@ -14,6 +14,11 @@
       k_step_begin, whose traffic is known exactly (the state read, Temp
       and the RK base written).  The table rows are
       `| group | kernel | fetch B | write B | traffic B |`.
+
+The face sweeps run in one launch of all directions, or, while their groups
+are timed, in one a direction; these launches have rows of their own, told
+apart by their order, and so have the updates that follow FP32 sweeps (see
+launches).  Batched sweeps (km_sweeps) are always of all directions.
 
 Run from fest-3d_amd/ (or with it on sys.path).
 """
@@ -29,7 +34,7 @@ from . import roofline as R
 
 
 GROUPS = [  # (substring of the demangled kernel name, kernel group)
-    ("k_sweeps<", "flux"),  # the three directions in one launch
+    ("k_sweeps<", "flux"),
     ("k_grad<", "grad"), ("k_mut_ghost_tp", "grad_bc"), ("k_update", "update"),
     ("k_bc_face", "bc_face"), ("k_bc_edges", "bc_edges"), ("k_step_begin", "step_begin"),
     ("k_dt_min", "time_step"), ("k_dt_fill", "time_step"), ("k_dt", "time_step"),
@@ -67,29 +72,61 @@ def _csvs(d, suffix):
     return out
 
 
+DIRECTIONS = ("i", "j", "k")
+
+
+def launches(rows):
+    """(group, kernel) of every dispatch of one run, by dispatch id.  rows:
+    (dispatch id, kernel name).  A residual runs the sweeps in one launch of all
+    directions or in three, i, j and k, one after the other, with other kernels
+    before and after.  An update after FP32 sweeps reads FP32 fluxes."""
+    rows = sorted(rows)
+    out, run, fp32 = {}, [], False
+    for n, name in rows + [(-1, "")]:
+        if name.startswith("k_sweeps<"):
+            fp32 = "float" in name
+            run.append((n, name))
+            continue
+        for e, (m, sweep) in enumerate(run):
+            d = DIRECTIONS[e % 3]
+            out[m] = ("flux_" + d, f"{sweep} {d}") if len(run) % 3 == 0 else ("flux", sweep + " all directions")
+        run = []
+        if name.startswith("km_sweeps<"):
+            fp32 = "float" in name
+        grp = group_of(name)
+        out[n] = (grp, name + " after float sweeps" if grp == "update" and fp32 else name)
+    return out
+
+
+def _dispatches(path):
+    """The rows of one CSV and the (group, kernel) of their dispatches."""
+    with open(path) as f:
+        rows = list(csv.DictReader(f))
+    return rows, launches({(int(r["Dispatch_Id"]), short(r["Kernel_Name"])) for r in rows})
+
+
 def stats(d):
-    rows = []
-    for path in _csvs(d, "kernel_stats.csv"):
-        with open(path) as f:
-            for r in csv.DictReader(f):
-                rows.append((short(r["Name"]), int(r["Calls"]), float(r["TotalDurationNs"]),
-                             float(r["AverageNs"]), float(r["Percentage"])))
-    rows.sort(key=lambda r: -r[2])
+    acc = defaultdict(list)
+    for path in _csvs(d, "kernel_trace.csv"):
+        rows, what = _dispatches(path)
+        for r in rows:
+            acc[what[int(r["Dispatch_Id"])]].append(float(r["End_Timestamp"]) - float(r["Start_Timestamp"]))
+    total = sum(sum(v) for v in acc.values())
     lines = ["| kernel | group | calls | avg us | total ms | % |", "|---|---|---|---|---|---|"]
-    for n, c, tot, avg, pct in rows:
-        lines.append(f"| {n} | {group_of(n)} | {c} | {avg / 1e3:.1f} | {tot / 1e6:.3f} | {pct:.1f} |")
+    for (grp, n), v in sorted(acc.items(), key=lambda kv: -sum(kv[1])):
+        t = sum(v)
+        lines.append(f"| {n} | {grp} | {len(v)} | {t / len(v) / 1e3:.1f} | {t / 1e6:.3f} | {100.0 * t / total:.1f} |")
     return "\n".join(lines)
 
 
 def counters(d, counter):
-    """Average counter value per dispatch, by kernel."""
+    """Average counter value per dispatch, by (group, kernel)."""
     acc = defaultdict(list)
     for path in _csvs(d, "counter_collection.csv"):
-        with open(path) as f:
-            for r in csv.DictReader(f):
-                if r.get("Counter_Name") != counter:
-                    continue
-                acc[short(r["Kernel_Name"])].append(float(r["Counter_Value"]))
+        rows, what = _dispatches(path)
+        for r in rows:
+            if r.get("Counter_Name") == counter:
+                acc[what[int(r["Dispatch_Id"])]].append(float(r["Counter_Value"]))
     return {k: sum(v) / len(v) for k, v in acc.items()}
 
 
@@ -126,12 +163,12 @@ def traffic(fetch_dir, write_dir, case_name):
              "",
              "| group | kernel | fetch B | write B | traffic B |", "|---|---|---|---|---|"]
     extra = ["", "| group | kernel | algorithmic B | traffic / algorithmic |", "|---|---|---|---|"]
-    for k in sorted(fe, key=lambda k: -fe[k]):
-        grp = group_of(k)
+    for key in sorted(fe, key=lambda k: -fe[k]):
+        grp, k = key
         if grp == "-":
             continue
-        f_b = fe[k] * 1024.0 * kf
-        w_b = wr.get(k, 0.0) * 1024.0 * kw
+        f_b = fe[key] * 1024.0 * kf
+        w_b = wr.get(key, 0.0) * 1024.0 * kw
         lines.append(f"| {grp} | {k} | {f_b:.4g} | {w_b:.4g} | {f_b + w_b:.6g} |")
         alg = R.bytes_per_launch(case, grp) if case is not None else None
         if alg:
@@ -147,16 +184,15 @@ def sq(d):
     instruction-cache hit rate when those counters were collected."""
     acc = defaultdict(lambda: defaultdict(list))
     for path in _csvs(d, "counter_collection.csv"):
-        with open(path) as f:
-            for r in csv.DictReader(f):
-                acc[short(r["Kernel_Name"])][r["Counter_Name"]].append(float(r["Counter_Value"]))
+        rows, what = _dispatches(path)
+        for r in rows:
+            acc[what[int(r["Dispatch_Id"])]][r["Counter_Name"]].append(float(r["Counter_Value"]))
     lines = ["| kernel | group | waves | VALU/wave | VALU busy | VMEM rd/wave | dep. wait | I-cache hit |",
              "|---|---|---|---|---|---|---|---|"]
-    for k in sorted(acc):
-        grp = group_of(k)
+    for grp, k in sorted(acc, key=lambda key: key[1]):
         if grp in ("setup", "-", "resnorm"):
             continue
-        m = {c: sum(v) / len(v) for c, v in acc[k].items()}
+        m = {c: sum(v) / len(v) for c, v in acc[grp, k].items()}
         waves = m.get("SQ_WAVES", 0.0)
 
         def fmt(x, f):

@@ -13,6 +13,10 @@ fest-3d_amd/csrc:
           with SST)
     write the face flux (n_var); the face sound speed at stage 1 (1, a
           quarter per launch over the four RK stages)
+  flux (k_sweeps of all three directions in one launch, as steps run it):
+    read  per cell q, the centre, the gradients, mu (+ mu_t, F1 with SST)
+          once, per face A,nx,ny,nz
+    write as above
   grad (k_grad<NG>, one thread per cell 0..imx x 0..jmx x 0..kmx):
     read  the n_grad gradient variables, volume, the i/j/k face metrics
           (3 x 4), rho and p when mu follows Sutherland, rho, dist and mu
@@ -102,6 +106,13 @@ def bytes_per_item(case, group):
 
 
 def bytes_per_launch(case, group):
+    if group == "flux":
+        # the three directions together: what a cell holds for all of them
+        # read once, each face's metrics and flux once
+        nv, sst = case.n_var, case.sst_family
+        cells = (case.imx - 1) * (case.jmx - 1) * (case.kmx - 1)
+        faces = sum(launch_items(case, "flux_" + d) for d in "ijk")
+        return W * (cells * (nv + 3 + 3 * _ngrad(case) + (3 if sst else 1)) + faces * (4 + nv + 0.25))
     n, b = launch_items(case, group), bytes_per_item(case, group)
     if n is None or b is None:
         return None
