@@ -191,12 +191,13 @@ __device__ __forceinline__ double sa_implicit(const Blk &b, long c, long gi, dou
 }
 
 // residue + SST/SA source, then (UPD_APPLY) the conservative update of the cell.
-// Bound by memory: 2.0 GB at 256 x 128 x 128 (SST) in 348 us, 5.8 TB/s.  What
-// the update needs is asked for ahead of the fluxes and those two variables
-// ahead of their sums, all of it with the variable count known at compile time;
-// one variable after another, each flux when its difference came up, took 355
-// us there, 7.9 us (now 4.7) at 64 x 64 x 4 and 64 us (now 43) over 24 blocks of
-// 1.1 M cells.
+// Bound by memory: 1.79 GB (a stage's average) at 256 x 128 x 128 (SST) in 345
+// us, 5.2 TB/s.  The stage's base state, R accumulator, source, volume and time
+// step are asked for ahead of the fluxes and those two variables ahead of their
+// sums, all of it with the variable count known at compile time; one variable
+// after another, each flux when its difference came up, took 355 us there, 7.9
+// us (now 4.7) at 64 x 64 x 4 and 64 us (now 43) over 24 blocks of 1.1 M cells.
+// What the turbulence models' implicit factors read follows the sums.
 template <int NV>
 __device__ __forceinline__ void k_update_b(const Blk &b, const Wg &wg, double TF, double SF, int flags) {
   int i, j;
@@ -214,9 +215,8 @@ __device__ __forceinline__ void k_update_b(const Blk &b, const Wg &wg, double TF
   const bool apply = flags & UPD_APPLY, more = apply && (flags & UPD_STORE) && !(flags & UPD_FIRST);
   const double *Qu = (flags & UPD_STORE) ? b.ust : b.qp;
   double R[NV], q0[NV], r0[NV], src[3] = {0.0, 0.0, 0.0};
-  double rho = 0.0, dt = 0.0, vol = 0.0;
+  double dt = 0.0, vol = 0.0;
   if (apply) {
-    rho = b.qp[c];
     dt = b.dt[r];
     vol = b.vol[c];
 #pragma unroll
