@@ -167,12 +167,13 @@ __device__ __forceinline__ bool tile_ij(int ni, int nj, int &i, int &j, int blk,
   j = ty * (256 >> lg) + ((int)threadIdx.x >> lg);
   return i < ni && j < nj;
 }
-// The tile width, at most `most`, that covers rows of ni cells, nj of them,
-// with the least work: the padded area, an eighth more for 32-wide tiles'
-// 16-wide ones, whose waves hold four rows (more of them next to a boundary,
-// shorter runs of memory).  97x61 cells take 64 (the sweeps 98 us at
-// 97x61x45 SST, 113 in 16-wide tiles), the 16..48-cell blocks of the chain 16
-// or 32 (211 -> 163 us).
+// The tile width, at most `most`, that covers rows of ni cells, nj of them, at
+// the least cost: the padded area, weighted by 1.03 for 32-wide and 1.16 for
+// 16-wide tiles, whose waves hold two and four rows (more of them next to a
+// boundary, shorter runs of memory).  The weights separate the two sets of
+// extents they were measured on: 97x61 cells take 64 (the sweeps 98 us at
+// 97x61x45 SST, 113 in 16-wide tiles), the 16..48-cell blocks of a chain 16 or
+// 32 (211 -> 163 us).
 inline int tile_width(int ni, int nj, int most) {
   int best = most;
   double cost = 0;

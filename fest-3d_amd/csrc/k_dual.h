@@ -65,7 +65,7 @@ struct Dual {
   friend __device__ __forceinline__ bool operator>=(const Dual &a, const Dual &b) { return a.v >= b.v; }
 
   // the face arithmetic's helpers (blk.h, k_flux.h) for dual arguments
-  // as operator/ with qdiv, for the quotients whose divisor is never zero
+  // as operator/ with qdiv, for divisors that are not subnormal
   friend __device__ __forceinline__ Dual tdiv(const Dual &a, const Dual &b) {
     Dual r;
     const double ib = qdiv(1.0, b.v);

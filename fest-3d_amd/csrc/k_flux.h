@@ -36,7 +36,7 @@ __device__ __forceinline__ double tsqrt(double x) { return sqrt(x); }
 __device__ __forceinline__ float tsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double tdiv(double a, double b) { return qdiv(a, b); }
 __device__ __forceinline__ float tdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-// quotients whose divisor may be zero
+// quotients of plain differences, whose divisor may be zero or subnormal
 __device__ __forceinline__ double xdiv(double a, double b) { return a / b; }
 __device__ __forceinline__ float xdiv(float a, float b) { return tdiv(a, b); }
 __device__ __forceinline__ double tabs(double x) { return fabs(x); }
@@ -542,8 +542,8 @@ struct FaceMath {
   // viscous flux's inputs one gradient ahead, all three sweeps of 256 x 128 x
   // 128 (SST, WENO5) take 1205 -> 1090 us, of 384 x 192 x 128 (PPM) 2630 ->
   // 2380 us; two or three variables ahead 1130 us, the gradients asked for
-  // before the inviscid flux 1175 us and up, with spills.  4.0 GB pass at 3.7
-  // TB/s then.  FP32 takes the stencils ahead too (256 x 128 x 128 760 -> 682 us,
+  // before the inviscid flux 1175 us and up, with spills.  3.5 GB pass at 3.3
+  // TB/s then, 2.2 GB needed.  FP32 takes the stencils ahead too (256 x 128 x 128 760 -> 682 us,
   // 24 blocks of 1.1 M cells, MUSCL, 163 -> 145 us; two variables ahead the
   // same); its viscous inputs fit the registers in the compiler's order (690 us
   // in this one).

@@ -557,7 +557,8 @@ __global__ void k_g32_widen(Blk b) {
 // A -11 face has no mu_t / F1 ghost rule (src/viscosity.f90:284-339,
 // 409-465 list -1..-9): its ghost cells keep the SST values
 // calculate_viscosity computes there, from the ghost gradients k_grad has
-// written (the FP32 ones where only those are kept).  Launched after it, only when an SST block has a -11 face.
+// written (the FP32 ones where only those are kept).  Launched after it, only
+// when an SST block has a -11 face.
 __device__ __forceinline__ void k_mut_ghost_tp_b(const Blk &b, const Wg &wg) {
   int face = wg.z;
   int a = wg.x * blockDim.x + threadIdx.x + 1;

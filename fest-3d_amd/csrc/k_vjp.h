@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(256) k_vjp_gather(Blk b, const double *__restr
 
 // the boundary face of `face` at (a, bb) (bnormal's face) in the compact
 // face order of its direction, and the I face whose normal the slip wall
-// reflects with (flow_tangency_col): compact I-face index, or -1 for the j
+// reflects with (k_bc_face_b, -6): compact I-face index, or -1 for the j
 // and k max faces, whose I face lies in the first ghost row
 __device__ __forceinline__ long vjp_bface(const Blk &b, int face, int a, int bb) {
   switch (face) {
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(256) k_vjp_bc(Blk b, int face0, double *bar, d
       long rf = -1;
       if (id == -6) {
         // u_g = u_c - 2 (n . u_c) r, n the boundary normal and r the
-        // I-face normal at the same index (flow_tangency_col)
+        // I-face normal at the same index (k_bc_face_b)
         bnormal(b, face, a, bb, nx, ny, nz);
         long f;
         switch (face) {

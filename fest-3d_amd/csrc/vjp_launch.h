@@ -32,12 +32,12 @@ struct VjpVisc {
 
 // bar (5 planes of the padded cell array) = d(barR . R)/dq on the resident
 // state, whose ghost cells the block's own boundary rules filled: the face
-// Jacobians contracted with barR (two launches), the per-cell
-// gather, then the transposes of the ghost rules in reverse face order, a
-// direction's two together where they touch different cells; with nodes.bar_nodes, also d(barR . R)/d(node coordinates).  With
-// visc.bt, the viscous faces' adjoints are added before the ghost rules'
-// transposes (the viscous faces reuse contrib after the gather: 22 planes).
-// contrib[d] holds vjp_contrib_len(b, d) doubles.
+// Jacobians contracted with barR (two launches), the per-cell gather, then the
+// transposes of the ghost rules in reverse face order, a direction's two
+// together where they touch different cells; with nodes.bar_nodes, also
+// d(barR . R)/d(node coordinates).  With visc.bt, the viscous faces' adjoints
+// are added before the ghost rules' transposes (the viscous faces reuse contrib
+// after the gather: 22 planes).  contrib[d] holds vjp_contrib_len(b, d) doubles.
 void launch_vjp(const Blk &b, hipStream_t st, const double *barR, double *const contrib[3], double *bar,
                 const VjpNodes &nodes, const VjpVisc &visc);
 
