@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <initializer_list>
+#include <mutex>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -65,6 +66,66 @@ struct StepGraphs {
   }
 };
 
+// Pinned host memory that kernels write a handle's norms and error word into:
+// the host reads them after one wait, without a transfer of their own.  Handles
+// take slots of shared 64 KiB pages, since a pinned allocation of each handle's
+// own costs 30 us and its release 100-220 us with other handles alive (a block of
+// 64 x 64 x 4 cells created and destroyed: 405 us, with slots 250-320).  A page
+// is released with its last slot, but for one that is kept; slots are handed
+// out under a lock, whichever thread or device the handle belongs to.
+namespace {
+constexpr size_t PINNED_SLOT = 256, PINNED_PAGE = 65536;
+constexpr int PINNED_SLOTS = (int)(PINNED_PAGE / PINNED_SLOT);
+static_assert(sizeof(double) * (NORM_SLOTS + 2) <= PINNED_SLOT, "a slot holds the norms and the error word");
+struct PinnedPage {
+  char *base;
+  std::vector<int> free;
+};
+struct Pinned {
+  std::mutex m;
+  std::vector<PinnedPage> pages;
+};
+Pinned &pinned() {
+  static Pinned *p = new Pinned;  // outlives every handle
+  return *p;
+}
+void *pinned_take() {
+  Pinned &P = pinned();
+  std::lock_guard<std::mutex> lock(P.m);
+  PinnedPage *page = nullptr;
+  for (PinnedPage &g : P.pages)
+    if (!g.free.empty()) page = &g;
+  if (!page) {
+    void *base = nullptr;
+    if (hipHostMalloc(&base, PINNED_PAGE, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) return nullptr;
+    P.pages.push_back(PinnedPage{(char *)base, {}});
+    page = &P.pages.back();
+    for (int n = PINNED_SLOTS - 1; n >= 0; --n) page->free.push_back(n);
+  }
+  const int n = page->free.back();
+  page->free.pop_back();
+  return page->base + n * PINNED_SLOT;
+}
+void pinned_give(void *slot) {
+  Pinned &P = pinned();
+  std::lock_guard<std::mutex> lock(P.m);
+  int unused = 0;
+  size_t mine = P.pages.size();
+  for (size_t g = 0; g < P.pages.size(); ++g) {
+    PinnedPage &page = P.pages[g];
+    if ((char *)slot >= page.base && (char *)slot < page.base + PINNED_PAGE) {
+      page.free.push_back((int)(((char *)slot - page.base) / PINNED_SLOT));
+      mine = g;
+    }
+    unused += (int)page.free.size() == PINNED_SLOTS;
+  }
+  if (unused > 1 && (int)P.pages[mine].free.size() == PINNED_SLOTS) {
+    (void)hipHostFree(P.pages[mine].base);
+    P.pages.erase(P.pages.begin() + (long)mine);
+  }
+}
+}  // namespace
+
 struct fest_handle {
   Blk b;
   hipStream_t stream = nullptr;      // the stream every launch goes to
@@ -78,9 +139,7 @@ struct fest_handle {
   std::vector<void *> allocs;
   long red_cap = 0;        // doubles in b.red
   int norm_blocks = 0;
-  // pinned host memory that kernels write the norms and the error word into:
-  // the host reads them after one wait, without a transfer of their own
-  double *host_norms = nullptr;    // NORM_SLOTS + 1
+  double *host_norms = nullptr;    // NORM_SLOTS + 1, a pinned slot
   unsigned *host_err = nullptr;
   bool have_grid = false, have_state = false;
   bool sk_geometry = false;  // the LU-SGS storage holds the current grid's geometry
@@ -950,10 +1009,8 @@ int fest_create(fest_handle **out, const fest_extent *dims, const fest_scheme *s
   if (hipMalloc(&e, sizeof(unsigned)) != hipSuccess) return fail(h, FEST_E_HIP, "hipMalloc(err)");
   h->allocs.push_back(e);
   b.err = (unsigned *)e;
-  void *pin = nullptr;
-  if (hipHostMalloc(&pin, sizeof(double) * (NORM_SLOTS + 2), hipHostMallocMapped) != hipSuccess)
-    return fail(h, FEST_E_HIP, "hipHostMalloc(norms)");
-  h->host_norms = (double *)pin;
+  h->host_norms = (double *)pinned_take();
+  if (!h->host_norms) return fail(h, FEST_E_HIP, "hipHostMalloc(norms)");
   h->host_err = (unsigned *)(h->host_norms + NORM_SLOTS + 1);
   HIPCHK(h, hipMemsetAsync(b.err, 0, sizeof(unsigned), h->stream));
   // molecular viscosity starts at mu_ref (src/viscosity.f90:565-568); F1 at 0
@@ -983,7 +1040,7 @@ void fest_destroy(fest_handle *h) {
   for (hipEvent_t e : h->ev_free) (void)hipEventDestroy(e);
   h->graphs.reset();
   for (void *p : h->allocs) (void)hipFree(p);
-  if (h->host_norms) (void)hipHostFree(h->host_norms);
+  if (h->host_norms) pinned_give(h->host_norms);
   if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
   delete h;
 }
@@ -1676,15 +1733,13 @@ int fest_group_create(fest_group **out, fest_handle *const *blocks, int nblocks,
   {
     std::vector<unsigned *> errs;
     for (int n = 0; n < nblocks; ++n) errs.push_back(blocks[n]->b.err);
-    void *pn = nullptr, *pe = nullptr;
+    void *p = nullptr;
     if (hipMalloc(&g->d_errs, sizeof(unsigned *) * nblocks) != hipSuccess ||
         hipMemcpy(g->d_errs, errs.data(), sizeof(unsigned *) * nblocks, hipMemcpyHostToDevice) != hipSuccess ||
-        hipHostMalloc(&pe, sizeof(unsigned) * nblocks, hipHostMallocMapped) != hipSuccess)
-      return gfail(g, FEST_E_HIP, "allocating the group's error words failed");
-    g->host_err = (unsigned *)pe;
-    if (hipHostMalloc(&pn, sizeof(double) * NORM_SLOTS * nblocks, hipHostMallocMapped) != hipSuccess)
-      return gfail(g, FEST_E_HIP, "allocating the group's norms failed");
-    g->host_norms = (double *)pn;
+        hipHostMalloc(&p, (sizeof(double) * NORM_SLOTS + sizeof(unsigned)) * nblocks, hipHostMallocMapped) != hipSuccess)
+      return gfail(g, FEST_E_HIP, "allocating the group's norms and error words failed");
+    g->host_norms = (double *)p;
+    g->host_err = (unsigned *)(g->host_norms + (size_t)NORM_SLOTS * nblocks);
   }
   if (hipStreamCreate(&g->stream) != hipSuccess) return gfail(g, FEST_E_HIP, "hipStreamCreate failed");
   for (int n = 0; n < nblocks; ++n) {
@@ -1788,7 +1843,6 @@ void fest_group_destroy(fest_group *g) {
   if (g->d_blks) (void)hipFree(g->d_blks);
   if (g->d_items) (void)hipFree(g->d_items);
   if (g->host_norms) (void)hipHostFree(g->host_norms);
-  if (g->host_err) (void)hipHostFree(g->host_err);
   if (g->d_errs) (void)hipFree(g->d_errs);
   for (fest_handle *h : g->blocks) {
     h->stream = h->own_stream;
